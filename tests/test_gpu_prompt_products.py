@@ -1,0 +1,47 @@
+"""Prompt passes' products (zh_pgemm.hip) in every format, at the edges of their tiles.
+
+A prompt's rows run through the products as tiles of 64, 128 or 256 tokens with the reduction split where
+few tiles would leave the chip idle.  Each model has one weight format, row counts off the 64- and 128-row
+tiles, and reductions of an even and an odd number of 256-value blocks; the prompts end one row before, on
+and after a tile's edge.  Logits within 1e-4 relative L2 and K/V rows within 1e-3 (one binary16 step) of
+the oracle's token-by-token prompt, as in test_gpu_prefill.py.
+"""
+import sys
+
+import numpy as np
+import pytest
+
+from oracle import zo
+from zhip import hip, synth
+from zhip.gguf import IQ4_XS, Q3_K, Q4_K, Q6_K, Q8_0, TYPE_NAMES
+
+pytestmark = pytest.mark.gpu
+
+
+def rel_l2(a, b):
+    b = np.asarray(b, np.float64)
+    return float(np.linalg.norm(np.asarray(a, np.float64) - b) / max(np.linalg.norm(b), 1e-30))
+
+
+@pytest.mark.parametrize("ttype", [Q4_K, Q6_K, Q8_0, IQ4_XS, Q3_K], ids=lambda t: TYPE_NAMES[t])
+# n rows in the pass: prompt - 1
+@pytest.mark.parametrize("rows", [17, 64, 65, 129, 257])
+def test_prompt_rows_match_the_token_by_token_prompt(hip_ctx, ttype, rows):
+    print(f"prompt products {TYPE_NAMES[ttype]} rows {rows}", flush=True)
+    sys.stdout.flush()
+    spec = synth.small_spec(hidden=512, ffn=768, n_head=4, n_kv=1, head_dim=64 if ttype == Q4_K else 128,
+                            default_type=ttype, attn_v_type=ttype, output_type=Q8_0, embd_type=Q8_0, context=300)
+    spec.n_head = 512 // spec.head_dim
+    img = synth.build(spec, seed=17)
+    prompt = synth.prompt_tokens(rows, rows + 1, spec.vocab)
+    o = zo.Session(zo.Model(img.buf), context=spec.context, kv_f16=True)
+    for t in prompt[:-1]:
+        o.step_no_output(int(t))
+    want = o.step(int(prompt[-1]))
+    s = hip.Session(hip_ctx, img, context=spec.context)
+    s.generate(prompt, 0)
+    assert rel_l2(s.logits(), want) < 1e-4
+    for pos in (0, rows // 2, rows - 1):
+        for a, b in zip(s.kv(1, pos), o.kv(1, pos)):
+            assert rel_l2(a, b) < 1e-3
+    s.close()

@@ -323,29 +323,37 @@ hipError_t launch_fill_u64(unsigned long long *p, unsigned long long v, int n, h
 // apart, max-ed into slots[row] (zero beforehand)
 hipError_t launch_argmax_rows(const float *x, int rows, int n, int ld, unsigned long long *slots, hipStream_t s);
 
-// Rows of activations split once for the exact-code GEMM (split_run16): row r
-// of the pieces at hi + r ld and lo + r ld, its 32-value sums at sum + r ld / 32
-// (ld a multiple of 32).  A producer writes them next to (or instead of the
-// GEMM re-splitting) its f32 rows; launch_gemm takes them as a hint.
-struct XPlanes {
-    uint16_t *hi, *lo;
-    float *sum;
-    int ld;
+// Rows of activations as the prompt products (zh_pgemm.hip) take them: each row
+// times a power of two that brings its largest magnitude to [2^14, 2^15), as
+// hi = binary16(v) and lo = binary16(v - hi) (v to 2^-22 relative, or 2^-40 of
+// the row's largest).  Slab kb holds values 32 kb .. of every row: x + (kb rows
+// + row) 64 is hi[32], lo[32].  xs: the 32-value sums / 64 of a 256-value block
+// as the same two pieces, xs + (block rows + row) 16.  scale: the inverse powers.
+struct HPlanes {
+    uint16_t *x, *xs;
+    float *scale;
 };
-// rows x n values of x (row stride ldx, n a multiple of 32) into xp
-hipError_t launch_split_rows(const float *x, int ldx, int rows, int n, const XPlanes &xp, hipStream_t s);
-// gate = silu(gate) * up (as launch_silu_mul, rows x n, row stride n), also into xp
-hipError_t launch_silu_mul_split(float *gate, const float *up, int rows, int n, const XPlanes &xp, hipStream_t s);
+// rows x n values of x (row stride ldx; n a multiple of 256) into xp
+hipError_t launch_row_planes(const float *x, int ldx, int rows, int n, const HPlanes &xp, hipStream_t s);
+// the rows' RMSNorm (as launch_rms_norm_rows) into xp, and into out where set
+hipError_t launch_norm_planes(const float *x, const float *w, float *out, int rows, int n, float eps, const HPlanes &xp,
+                              hipStream_t s);
+// Products of many token rows with up to three matrices of one quantized
+// format and row size: OUT_STORE, OUT_ADD, or OUT_SWIGLU with w2 (one matrix).
+// part: workspace for the partial results of a split reduction (added in a
+// fixed order: the same inputs give the same bits).
+bool pgemm_supported(int fmt, int K, const void *w, uint64_t stride);
+hipError_t launch_pgemm(int fmt, int nseg, const uint8_t *const *w, const uint8_t *w2, float *const *y, const int *ldy,
+                        const int *N, uint64_t stride, const HPlanes &xp, int M, int K, int out, float *part,
+                        size_t part_floats, hipStream_t s, int force_cfg = -1, int force_ks = 0);
 // MFMA GEMM for M >= 8 tokens (zh_gemm.hip): Y[m][n] (=, +=) sum_k W[n][k] X[m][k]
 // (OUT_STORE / OUT_ADD / OUT_SWIGLU with w2 / OUT_ARGMAX into argmax[M]).
 // max_split bounds the reduction split of the exact-code kernel, whose
 // partial results add atomically: 1 keeps a += product deterministic, 2 a
 // product into a cleared output (0 + a + b is the same in either order).
-// xp (optional): the same input already split (XPlanes), used when the
-// exact-code kernel runs.
 hipError_t launch_gemm(int fmt, const uint8_t *w, const uint8_t *w2, uint64_t stride, const float *x, int ldx,
                        float *y, int ldy, int M, int N, int K, int out, unsigned long long *argmax, hipStream_t s,
-                       bool precise = false, int max_split = 16, const XPlanes *xp = nullptr);
+                       bool precise = false, int max_split = 16);
 // The deferred RMSNorm of a product's input rows (rmsNorm, model/loader.zig:
 // 3404-3426, with its scale moved past the product): the product takes
 // x * w, and each row's sum of squares of x is added to ss[row] (when ss is
@@ -360,15 +368,12 @@ struct RowNorm {
 // the deferred norm of the input.
 hipError_t launch_gemm_multi(int fmt, int nseg, const uint8_t *const *w, float *const *y, const int *ldy,
                              const int *N, uint64_t stride, const float *x, int ldx, int M, int K, int out,
-                             hipStream_t s, int max_split = 16, const XPlanes *xp = nullptr,
-                             const RowNorm *rn = nullptr);
+                             hipStream_t s, int max_split = 16, const RowNorm *rn = nullptr);
 // whether launch_gemm_multi takes a RowNorm for these matrices
 bool gemm_rownorm_supported(int fmt, int K, const void *w, uint64_t stride);
-// xp (optional): the normed rows also split into xp (as launch_split_rows),
-// in the same launch where the row fits.
 hipError_t launch_rms_norm_rows(const float *x, const float *w, float *out, int rows, int n, float eps, hipStream_t s,
                                 float *clear0 = nullptr, size_t n0 = 0, float *clear1 = nullptr, size_t n1 = 0,
-                                float *clear2 = nullptr, size_t n2 = 0, const XPlanes *xp = nullptr);
+                                float *clear2 = nullptr, size_t n2 = 0);
 // Grouped by expert (MoE prefill): token tiles from launch_moe_group; W of expert e
 // starts expert_stride bytes after W of expert e - 1; x row = id / x_div, y row = id.
 hipError_t launch_gemm_grouped(int fmt, const uint8_t *w, const uint8_t *w2, uint64_t stride, uint64_t expert_stride,
@@ -378,13 +383,13 @@ hipError_t launch_gemm_grouped(int fmt, const uint8_t *w, const uint8_t *w2, uin
 bool qgemm_supported(int fmt, int K, const void *w, const void *w2, uint64_t stride, uint64_t expert_stride);
 hipError_t launch_qgemm(int fmt, const uint8_t *w, const uint8_t *w2, uint64_t stride, const float *x, int ldx,
                         float *y, int ldy, int M, int N, int K, int out, unsigned long long *argmax, hipStream_t s,
-                        int max_split = 16, const XPlanes *xp = nullptr);
+                        int max_split = 16);
 // Up to three matrices of one format, row stride and reduction length against
 // one input in one launch (matrix i: rows N[i], output y[i] with row stride ldy[i]).
 hipError_t launch_qgemm_multi(int fmt, int nseg, const uint8_t *const *w, float *const *y, const int *ldy,
                               const int *N, const uint8_t *w2, uint64_t stride, const float *x, int ldx, int M, int K,
                               int out, unsigned long long *argmax, hipStream_t s, int max_split = 16,
-                              const XPlanes *xp = nullptr, const RowNorm *rn = nullptr);
+                              const RowNorm *rn = nullptr);
 hipError_t launch_qgemm_grouped(int fmt, const uint8_t *w, const uint8_t *w2, uint64_t stride,
                                 uint64_t expert_stride, const float *x, int ldx, int x_div, float *y, int ldy, int N,
                                 int K, int out, const int *tiles, const int *list, const int *ntiles, int max_tiles,

@@ -48,8 +48,9 @@ struct ZiggyHipMoeStack {
     // prefill (token batches of up to pre_max rows), allocated at the first call
     int pre_max = 0;
     float *p_input = nullptr, *p_hidden = nullptr, *p_normed = nullptr, *p_logits = nullptr, *p_act = nullptr,
-          *p_act_sh = nullptr, *p_tmp = nullptr, *p_sh = nullptr, *p_up_sh = nullptr;
-    zh::XPlanes p_xp{};  // the shared expert's inputs, split once per layer
+          *p_act_sh = nullptr, *p_tmp = nullptr, *p_sh = nullptr;
+    zh::HPlanes p_hp{};  // the shared expert's inputs as planes, and its products' workspace
+    float *p_part = nullptr;
     uint32_t *p_route = nullptr;  // [layers][pre_max][2k + 2]
     int *p_list = nullptr, *p_tiles = nullptr, *p_ntiles = nullptr;
 };
@@ -272,18 +273,29 @@ hipError_t enqueue_layer(ZiggyHipMoeStack *s, int l, hipStream_t st) {
 //   gate/up  grouped SWIGLU GEMM -> p_act[t * k + s]; shared -> p_act_sh[t]
 //   down     grouped GEMM -> p_tmp[t * k + s]; shared -> p_sh[t]
 //   combine  per row, slot order as in decode
+constexpr size_t kSharedPart = 4u << 20;  // floats of the shared products' split workspace
 hipError_t enqueue_prefill_layer(ZiggyHipMoeStack *s, int l, int M, hipStream_t st) {
     const MoeLayerW &L = s->layers[l];
     const ZiggyHipMoeDesc &d = s->d;
     const int H = (int)d.hidden, E = (int)d.expert_count, K = (int)d.expert_used_count, FF = (int)d.expert_ff_length,
               SF = (int)d.shared_ff_length;
     uint32_t *route = s->p_route + (size_t)l * s->pre_max * s->route_stride;
-    // the shared expert on split inputs (more than one token tile): the norm
-    // also splits its rows; gate and up as two stores in one launch, then
-    // SiLU * up split for down
-    const bool sh_split = s->shared && M > 16 && H % 32 == 0 && SF % 32 == 0 && s->p_xp.hi;
-    hipError_t e = launch_rms_norm_rows(s->p_hidden, (const float *)L.norm.p, s->p_normed, M, H, d.rms_norm_eps, st,
-                                        nullptr, 0, nullptr, 0, nullptr, 0, sh_split ? &s->p_xp : nullptr);
+    // the shared expert from planes (more than one token tile): the norm
+    // writes its rows' planes too; gate, up and SiLU * up in one launch
+    auto pg_ok = [](const DT &w) { return pgemm_supported((int)w.type, (int)w.cols, w.p, w.stride); };
+    const bool sh_planes = s->shared && M > 16 && s->p_hp.x && pg_ok(L.gate_sh) && pg_ok(L.up_sh) && pg_ok(L.down_sh) &&
+                           L.gate_sh.type == L.up_sh.type;
+    hipError_t e = sh_planes ? launch_norm_planes(s->p_hidden, (const float *)L.norm.p, s->p_normed, M, H, d.rms_norm_eps,
+                                                  s->p_hp, st)
+                             : launch_rms_norm_rows(s->p_hidden, (const float *)L.norm.p, s->p_normed, M, H,
+                                                    d.rms_norm_eps, st);
+    auto sh_product = [&](const DT &w, const DT *w2, float *y, int n, int out) {
+        const uint8_t *ws[1] = {w.p};
+        float *ys[1] = {y};
+        const int Ns[1] = {n};
+        return launch_pgemm((int)w.type, 1, ws, w2 ? w2->p : nullptr, ys, Ns, Ns, w.stride, s->p_hp, M, (int)w.cols, out,
+                            s->p_part, kSharedPart, st);
+    };
     // the shared gate row, stored right after the router's rows, is row E of one launch
     const bool gate_row_next = s->shared_gate && L.gate_inp_sh.p == L.router.p + (uint64_t)E * L.router.stride &&
                                L.gate_inp_sh.stride == L.router.stride;
@@ -303,14 +315,10 @@ hipError_t enqueue_prefill_layer(ZiggyHipMoeStack *s, int l, int M, hipStream_t 
         e = launch_gemm_grouped(L.gate.type, L.gate.p, L.up.p, L.gate.stride, (uint64_t)FF * L.gate.stride,
                                 s->p_normed, H, K, s->p_act, FF, FF, H, OUT_SWIGLU, s->p_tiles, s->p_list,
                                 s->p_ntiles, max_tiles, st);
-    if (e == hipSuccess && sh_split) {
-        const uint8_t *ws[2] = {L.gate_sh.p, L.up_sh.p};
-        float *ys[2] = {s->p_act_sh, s->p_up_sh};
-        const int lds[2] = {SF, SF}, Ns[2] = {SF, SF};
-        if (e == hipSuccess)
-            e = launch_gemm_multi(L.gate_sh.type, 2, ws, ys, lds, Ns, L.gate_sh.stride, s->p_normed, H, M, H,
-                                  OUT_STORE, st, 1, &s->p_xp);
-        if (e == hipSuccess) e = launch_silu_mul_split(s->p_act_sh, s->p_up_sh, M, SF, s->p_xp, st);
+    if (e == hipSuccess && sh_planes) {
+        e = sh_product(L.gate_sh, &L.up_sh, s->p_act_sh, SF, OUT_SWIGLU);
+        if (e == hipSuccess) e = launch_row_planes(s->p_act_sh, SF, M, SF, s->p_hp, st);
+        if (e == hipSuccess) e = sh_product(L.down_sh, nullptr, s->p_sh, H, OUT_STORE);
     } else if (e == hipSuccess && s->shared) {
         e = launch_gemm(L.gate_sh.type, L.gate_sh.p, L.up_sh.p, L.gate_sh.stride, s->p_normed, H, s->p_act_sh, SF, M,
                         SF, H, OUT_SWIGLU, nullptr, st);
@@ -319,9 +327,9 @@ hipError_t enqueue_prefill_layer(ZiggyHipMoeStack *s, int l, int M, hipStream_t 
         e = launch_gemm_grouped(L.down.type, L.down.p, nullptr, L.down.stride, (uint64_t)H * L.down.stride, s->p_act,
                                 FF, 1, s->p_tmp, H, H, FF, OUT_STORE, s->p_tiles, s->p_list, s->p_ntiles, max_tiles,
                                 st);
-    if (e == hipSuccess && s->shared)
+    if (e == hipSuccess && s->shared && !sh_planes)
         e = launch_gemm(L.down_sh.type, L.down_sh.p, nullptr, L.down_sh.stride, s->p_act_sh, SF, s->p_sh, H, M, H, SF,
-                        OUT_STORE, nullptr, st, false, 16, sh_split ? &s->p_xp : nullptr);
+                        OUT_STORE, nullptr, st);
     if (e == hipSuccess)
         e = launch_moe_combine(s->p_hidden, s->p_tmp, route, H, K, s->shared ? 1 : 0, st, M,
                                s->shared ? s->p_sh : nullptr);
@@ -345,7 +353,6 @@ hipError_t prefill_alloc(ZiggyHipMoeStack *s) {
         {(void **)&s->p_logits, Mc * (E + 1) * 4},
         {(void **)&s->p_act, Mc * K * FF * 4},
         {(void **)&s->p_act_sh, Mc * (SF ? SF : 1) * 4},
-        {(void **)&s->p_up_sh, Mc * (SF ? SF : 1) * 4},
         {(void **)&s->p_tmp, Mc * K * H * 4},
         {(void **)&s->p_sh, Mc * H * 4},
         {(void **)&s->p_route, NL * Mc * s->route_stride * 4},
@@ -359,16 +366,20 @@ hipError_t prefill_alloc(ZiggyHipMoeStack *s) {
         if (e != hipSuccess) return e;
         s->allocs.push_back(*r.p);
     }
-    {
-        const size_t ld = (std::max(H, SF) + 31) / 32 * 32;
-        uint8_t *base = nullptr;
-        hipError_t e = hipMalloc((void **)&base, Mc * ld * 4 + Mc * (ld / 32) * 4);
-        if (e != hipSuccess) return e;
-        s->allocs.push_back(base);
-        s->p_xp.hi = reinterpret_cast<uint16_t *>(base);
-        s->p_xp.lo = s->p_xp.hi + Mc * ld;
-        s->p_xp.sum = reinterpret_cast<float *>(s->p_xp.lo + Mc * ld);
-        s->p_xp.ld = (int)ld;
+    if (s->shared) {
+        const size_t nblk = std::max(H, SF) / 256 + 1;
+        struct {
+            void **p;
+            size_t bytes;
+        } planes[] = {{(void **)&s->p_hp.xs, Mc * nblk * 32},
+                      {(void **)&s->p_hp.scale, Mc * 4},
+                      {(void **)&s->p_part, kSharedPart * 4},
+                      {(void **)&s->p_hp.x, Mc * nblk * 256 * 4}};
+        for (auto &r : planes) {
+            hipError_t e = hipMalloc(r.p, r.bytes);
+            if (e != hipSuccess) return e;
+            s->allocs.push_back(*r.p);
+        }
     }
     s->pre_max = (int)Mc;
     return hipSuccess;

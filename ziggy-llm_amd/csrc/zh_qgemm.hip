@@ -70,11 +70,6 @@ struct QGemmParams {
     const uint8_t *ws[2];
     float *ys[2];
     int Ns[2], ldys[2], gs[2];
-    // the input already split (XPlanes; the XP kernels): row r's pieces at
-    // xh / xl + r ldxs, its 32-value sums at xsum + r ldxs / 32
-    const uint16_t *xh, *xl;
-    const float *xsum;
-    int ldxs;
     // NRM kernels: the deferred RMSNorm of the input rows -- the products take
     // x * norm_w (per reduction index), and the row's sum of squares of x
     // over this reduction range adds to row_ss[row] (one workgroup per range)
@@ -322,10 +317,10 @@ template <> struct QChunk<Q3_K> {
 // Geometry of the kernel for format F (two matrices for SWIGLU).  A chunk row
 // at any offset kShm allows lies in kWin 16-byte windows; its LDS image has
 // one spare window (a word read past the last byte) and an odd window count,
-// so the 16 rows' words fall in distinct banks.  The activation stage (TT
-// token tiles of 16) is as long as LDS allows next to the code images (2048,
+// so the 16 rows' words fall in distinct banks.  The activation stage (16
+// tokens) is as long as LDS allows next to the code images (2048,
 // 1024 or 512 values).
-template <int F, bool kPair, int TT = 1, int OCC = 1> struct QGeom {
+template <int F, bool kPair, int OCC = 1> struct QGeom {
     static constexpr int kMats = kPair ? 2 : 1;
     static constexpr int kWin = (QChunk<F>::kCB + QChunk<F>::kShm + 15) / 16;
     static constexpr int kRowW = 4 * ((kWin + 1) | 1);
@@ -336,7 +331,7 @@ template <int F, bool kPair, int TT = 1, int OCC = 1> struct QGeom {
     // activation rows of st + 8 values (the last without its padding), the
     // sums, the code images
     static constexpr int lds_bytes(int st) {
-        return 2 * ((2 * 16 * TT - 1) * (st + 8) + st) + (kXsum ? st / QChunk<F>::kSub * 16 * TT * 4 : 4) + kCodeBytes;
+        return 2 * ((2 * 16 - 1) * (st + 8) + st) + (kXsum ? st / QChunk<F>::kSub * 16 * 4 : 4) + kCodeBytes;
     }
     // OCC > 1: the longest stage that leaves LDS for OCC workgroups per CU
     // (one stages or waits while another computes), where one fits
@@ -356,18 +351,15 @@ __device__ __forceinline__ uint32_t ordered_bits_q(float v) {
     return (b & 0x80000000u) ? ~b : (b | 0x80000000u);
 }
 
-// XP: the input comes split (XPlanes) and a workgroup takes two token tiles
-// (32 tokens): every decoded code serves both tiles' products.
-template <int F, int OUT, bool GROUPED, int R, bool XP, bool NRM = false>
+template <int F, int OUT, bool GROUPED, int R, bool NRM = false>
 __global__ void __launch_bounds__(256, OUT != OUT_SWIGLU ? 2 : 1) qgemm_kernel(QGemmParams p) {
-    static_assert(!NRM || (!XP && !GROUPED), "the deferred norm stages plain rows");
+    static_assert(!NRM || !GROUPED, "the deferred norm stages plain rows");
     constexpr bool kPair = OUT == OUT_SWIGLU;
-    constexpr int TT = XP ? 2 : 1;  // token tiles of 16 per workgroup
     // LDS for two workgroups per CU (three for the grouped single products,
     // whose registers allow it; one for the dense SWIGLU pair)
-    constexpr int OCC = GROUPED && !kPair ? 3 : XP || GROUPED || !kPair ? 2 : 1;
+    constexpr int OCC = GROUPED && !kPair ? 3 : GROUPED || !kPair ? 2 : 1;
     using QC = QChunk<F>;
-    using G = QGeom<F, kPair, TT, OCC>;
+    using G = QGeom<F, kPair, OCC>;
     constexpr int kSub = QC::kSub, kCB = QC::kCB, kShm = QC::kShm;
     constexpr int kMats = G::kMats, kWin = G::kWin, kRowW = G::kRowW, kPieces = G::kPieces, kP = G::kP;
     constexpr bool kXsum = G::kXsum;
@@ -379,7 +371,7 @@ __global__ void __launch_bounds__(256, OUT != OUT_SWIGLU ? 2 : 1) qgemm_kernel(Q
 
     touch_params(p);
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, li = lane & 15, lg = lane >> 4;
-    int m0 = blockIdx.y * 16 * TT, M = p.M;
+    int m0 = blockIdx.y * 16, M = p.M;
     const int *ids = nullptr;
     const uint8_t *w = p.w, *w2 = p.w2;
     if (GROUPED) {
@@ -424,10 +416,10 @@ __global__ void __launch_bounds__(256, OUT != OUT_SWIGLU ? 2 : 1) qgemm_kernel(Q
         ca = cb + tc - gi * nspan;
     };
 
-    // The activations of a stage (up to kStage values of all 16 TT tokens)
+    // The activations of a stage (up to kStage values of all 16 tokens)
     // sit in LDS as bf16 hi / lo pieces; thread (token tt, part) stages values
-    // 16 part + 256 i of tokens tt, tt + 16, ...
-    constexpr int NT = 16 * TT;
+    // 16 part + 256 i of token tt
+    constexpr int NT = 16;
     // [hi / lo][token][k]: rows kStage + 8 apart (the padding spreads the
     // rows' words over the banks), the last row without its padding
     constexpr int kXRow = kStage + 8;
@@ -436,192 +428,131 @@ __global__ void __launch_bounds__(256, OUT != OUT_SWIGLU ? 2 : 1) qgemm_kernel(Q
     __shared__ __align__(16) float xsum_s[kXsum ? kStage / kSub : 1][kXsum ? NT : 1];  // [sub-block][token]: -kOff X
     __shared__ __align__(16) uint32_t code_s[4][kMats][16 * kRowW];        // [wavefront][matrix][row image]
     const int tt = tid >> 4, part = tid & 15;
-    static_assert(!XP || !kXsum || kSub == 32, "split inputs carry 32-value sums");
-    bool tok_ok[TT];
-    const float *xrow[TT];
+    const bool tok_ok = m0 + tt < M;
     const float *nwrow = NRM ? p.norm_w + 16 * part : nullptr;
     float ssq = 0.f;  // NRM: this thread's sum of squares of its token's staged values
-    const uint16_t *xhrow[TT], *xlrow[TT];
-    const float *xsrow[TT];
-#pragma unroll
-    for (int t = 0; t < TT; t++) {
-        tok_ok[t] = m0 + 16 * t + tt < M;
-        const int m = min(m0 + 16 * t + tt, M - 1);
-        const size_t r = (size_t)(GROUPED ? ids[m] / p.x_div : m);
-        xrow[t] = p.x + r * p.ldx + 16 * part;
-        if (XP) {
-            xhrow[t] = p.xh + r * p.ldxs + 16 * part;
-            xlrow[t] = p.xl + r * p.ldxs + 16 * part;
-            xsrow[t] = p.xsum + r * (p.ldxs / 32) + (part >> 1);
-        }
-    }
+    const int mrow = min(m0 + tt, M - 1);
+    const float *xrow = p.x + (size_t)(GROUPED ? ids[mrow] / p.x_div : mrow) * p.ldx + 16 * part;
     // stage_load issues the whole stage's activation loads (clamped to its
     // last chunk: unconditional, so the compiler's wait counting stays exact)
     // into ld; stage_store splits every chunk and writes those of the stage.
-    // XP: the pieces and sums as split by the producer (tokens past M repeat
-    // the last row; their results are never stored).
-    float4 ld[TT][kStageChunks][4];
+    float4 ld[kStageChunks][4];
     float4 ldw[NRM ? kStageChunks : 1][4];
-    float lsum[TT][XP ? kStageChunks : 1];
     auto stage_load = [&](int kb, int nc) {
 #pragma unroll
-        for (int t = 0; t < TT; t++)
+        for (int u = 0; u < kStageChunks; u++) {
+            const int ko = kb + min(u, nc - 1) * kQChunk;
+            const float4 *src = reinterpret_cast<const float4 *>(xrow + ko);
 #pragma unroll
-            for (int u = 0; u < kStageChunks; u++) {
-                const int ko = kb + min(u, nc - 1) * kQChunk;
-                if constexpr (XP) {
-                    const float4 *h = reinterpret_cast<const float4 *>(xhrow[t] + ko);
-                    const float4 *l = reinterpret_cast<const float4 *>(xlrow[t] + ko);
-                    ld[t][u][0] = h[0];
-                    ld[t][u][1] = h[1];
-                    ld[t][u][2] = l[0];
-                    ld[t][u][3] = l[1];
-                    if (kXsum) lsum[t][XP ? u : 0] = xsrow[t][ko / 32];
-                } else {
-                    const float4 *src = reinterpret_cast<const float4 *>(xrow[t] + ko);
+            for (int i = 0; i < 4; i++) ld[u][i] = src[i];
+            if (NRM) {
+                const float4 *nw = reinterpret_cast<const float4 *>(nwrow + ko);
 #pragma unroll
-                    for (int i = 0; i < 4; i++) ld[t][u][i] = src[i];
-                    if (NRM && t == 0) {
-                        const float4 *nw = reinterpret_cast<const float4 *>(nwrow + ko);
-#pragma unroll
-                        for (int i = 0; i < 4; i++) ldw[u][i] = nw[i];
-                    }
-                }
+                for (int i = 0; i < 4; i++) ldw[u][i] = nw[i];
             }
+        }
     };
     auto stage_store = [&](int nc) {
 #pragma unroll
-        for (int t = 0; t < TT; t++)
+        for (int u = 0; u < kStageChunks; u++) {
+            if (u >= nc) {
+                // past the range: the loads still land -- consumed here, so the
+                // compiler's wait counting sees them complete on every path
 #pragma unroll
-            for (int u = 0; u < kStageChunks; u++) {
-                if (u >= nc) {
-                    // past the range: the loads still land -- consumed here, so the
-                    // compiler's wait counting sees them complete on every path
+                for (int i = 0; i < 4; i++)
+                    __asm__ volatile("" ::"v"(ld[u][i].x), "v"(ld[u][i].y), "v"(ld[u][i].z), "v"(ld[u][i].w));
+                if (NRM)
 #pragma unroll
                     for (int i = 0; i < 4; i++)
-                        __asm__ volatile("" ::"v"(ld[t][u][i].x), "v"(ld[t][u][i].y), "v"(ld[t][u][i].z),
-                                         "v"(ld[t][u][i].w));
-                    if (XP && kXsum) __asm__ volatile("" ::"v"(lsum[t][XP ? u : 0]));
-                    if (NRM && t == 0)
-#pragma unroll
-                        for (int i = 0; i < 4; i++)
-                            __asm__ volatile("" ::"v"(ldw[u][i].x), "v"(ldw[u][i].y), "v"(ldw[u][i].z),
-                                             "v"(ldw[u][i].w));
-                    continue;
-                }
-                uint32_t hw[8], lw[8];
-                float sum = 0.f;
-                if constexpr (XP) {
-                    // the loaded words are the pieces: hi of values 0..15, then lo
-                    __builtin_memcpy(hw, &ld[t][u][0], 32);
-                    __builtin_memcpy(lw, &ld[t][u][2], 32);
-                    if (kXsum) sum = lsum[t][XP ? u : 0];
-                } else {
-                    float v[16];
-#pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        v[4 * i] = tok_ok[t] ? ld[t][u][i].x : 0.f;
-                        v[4 * i + 1] = tok_ok[t] ? ld[t][u][i].y : 0.f;
-                        v[4 * i + 2] = tok_ok[t] ? ld[t][u][i].z : 0.f;
-                        v[4 * i + 3] = tok_ok[t] ? ld[t][u][i].w : 0.f;
-                    }
-                    if constexpr (NRM) {
-                        // rmsNorm's (scale x) w with the scale deferred to the
-                        // product's reader: the sum of squares of x, then x w
-#pragma unroll
-                        for (int i = 0; i < 16; i++) ssq = fmaf(v[i], v[i], ssq);
-#pragma unroll
-                        for (int i = 0; i < 4; i++) {
-                            v[4 * i] *= ldw[u][i].x, v[4 * i + 1] *= ldw[u][i].y;
-                            v[4 * i + 2] *= ldw[u][i].z, v[4 * i + 3] *= ldw[u][i].w;
-                        }
-                    }
-                    sum = split_run16(v, hw, lw);
-                    if (kXsum && kSub == 32) sum += __shfl_xor(sum, 1, 64);  // the other half of the 32-value sub-block
-                }
-                const int tk = 16 * t + tt;
-                uint4 *dh = reinterpret_cast<uint4 *>(xs_at(0, tk, u * kQChunk + 16 * part));
-                uint4 *dl = reinterpret_cast<uint4 *>(xs_at(1, tk, u * kQChunk + 16 * part));
-                dh[0] = {hw[0], hw[1], hw[2], hw[3]};
-                dh[1] = {hw[4], hw[5], hw[6], hw[7]};
-                dl[0] = {lw[0], lw[1], lw[2], lw[3]};
-                dl[1] = {lw[4], lw[5], lw[6], lw[7]};
-                if (kXsum && kSub == 32 && !(part & 1)) xsum_s[u * 8 + (part >> 1)][tk] = -QC::kOff * sum;
-                if (kXsum && kSub == 16) xsum_s[u * 16 + part][tk] = -QC::kOff * sum;
+                        __asm__ volatile("" ::"v"(ldw[u][i].x), "v"(ldw[u][i].y), "v"(ldw[u][i].z), "v"(ldw[u][i].w));
+                continue;
             }
+            uint32_t hw[8], lw[8];
+            float v[16];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                v[4 * i] = tok_ok ? ld[u][i].x : 0.f;
+                v[4 * i + 1] = tok_ok ? ld[u][i].y : 0.f;
+                v[4 * i + 2] = tok_ok ? ld[u][i].z : 0.f;
+                v[4 * i + 3] = tok_ok ? ld[u][i].w : 0.f;
+            }
+            if constexpr (NRM) {
+                // rmsNorm's (scale x) w with the scale deferred to the
+                // product's reader: the sum of squares of x, then x w
+#pragma unroll
+                for (int i = 0; i < 16; i++) ssq = fmaf(v[i], v[i], ssq);
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    v[4 * i] *= ldw[u][i].x, v[4 * i + 1] *= ldw[u][i].y;
+                    v[4 * i + 2] *= ldw[u][i].z, v[4 * i + 3] *= ldw[u][i].w;
+                }
+            }
+            float sum = split_run16(v, hw, lw);
+            if (kXsum && kSub == 32) sum += __shfl_xor(sum, 1, 64);  // the other half of the 32-value sub-block
+            uint4 *dh = reinterpret_cast<uint4 *>(xs_at(0, tt, u * kQChunk + 16 * part));
+            uint4 *dl = reinterpret_cast<uint4 *>(xs_at(1, tt, u * kQChunk + 16 * part));
+            dh[0] = {hw[0], hw[1], hw[2], hw[3]};
+            dh[1] = {hw[4], hw[5], hw[6], hw[7]};
+            dl[0] = {lw[0], lw[1], lw[2], lw[3]};
+            dl[1] = {lw[4], lw[5], lw[6], lw[7]};
+            if (kXsum && kSub == 32 && !(part & 1)) xsum_s[u * 8 + (part >> 1)][tt] = -QC::kOff * sum;
+            if (kXsum && kSub == 16) xsum_s[u * 16 + part][tt] = -QC::kOff * sum;
+        }
     };
 
-    qf4v acc[TT], acc2[TT];
-#pragma unroll
-    for (int t = 0; t < TT; t++) acc[t] = acc2[t] = qf4v{0.f, 0.f, 0.f, 0.f};
+    qf4v acc = {0.f, 0.f, 0.f, 0.f}, acc2 = {0.f, 0.f, 0.f, 0.f};
     // chunk cs of the stage (offset 256 cs in LDS)
     // All products of the chunk first (independent accumulators, so the
-    // matrix core pipelines them), then the scales.  A step's codes are
-    // decoded once for the TT token tiles.
+    // matrix core pipelines them), then the scales.
     auto compute = [&](const QC &r, const QC &r2, int cs, float live) {
         constexpr int S = QC::kSteps;
-        // steps per pass: the products of at most 16 (step, tile) pairs in registers
-        constexpr int P = S * TT > 16 ? 16 / TT : S;
         const qf4v zero = {0.f, 0.f, 0.f, 0.f};
-        qf4v dv[TT][S], dv2[TT][S];
+        qf4v dv[S], dv2[S];
         float sv[S], sv2[S];
 #pragma unroll
-        for (int j0 = 0; j0 < S; j0 += P) {
-#pragma unroll
-        for (int j = j0; j < j0 + P; j++) {
+        for (int j = 0; j < S; j++) {
             sv2[j] = 0.f;
             const int kx = cs * kQChunk + kSub * j;
+            dv2[j] = zero;
             if constexpr (kSub == 32) {
                 const bf8v b = as_bf8(r.step(j, sv[j]));
                 bf8v b2 = b;
                 if (kPair) b2 = as_bf8(r2.step(j, sv2[j]));
-#pragma unroll
-                for (int t = 0; t < TT; t++) {
-                    const bf8v ah = as_bf8(*reinterpret_cast<const uint4 *>(xs_at(0, 16 * t + li, kx + 8 * lg)));
-                    const bf8v al = as_bf8(*reinterpret_cast<const uint4 *>(xs_at(1, 16 * t + li, kx + 8 * lg)));
-                    // kOff codes: the products start from -kOff X (the staged
-                    // sums of tokens 4 lg .. 4 lg + 3), so the code offset
-                    // cancels inside the product: D, not D + kOff X
-                    qf4v c0 = zero;
-                    if constexpr (kXsum)
-                        c0 = *reinterpret_cast<const qf4v *>(&xsum_s[cs * (kQChunk / kSub) + j][16 * t + 4 * lg]);
-                    dv[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, b, c0, 0, 0, 0);
-                    dv[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, b, dv[t][j], 0, 0, 0);
-                    dv2[t][j] = zero;
-                    if (kPair) {
-                        dv2[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, b2, c0, 0, 0, 0);
-                        dv2[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, b2, dv2[t][j], 0, 0, 0);
-                    }
+                const bf8v ah = as_bf8(*reinterpret_cast<const uint4 *>(xs_at(0, li, kx + 8 * lg)));
+                const bf8v al = as_bf8(*reinterpret_cast<const uint4 *>(xs_at(1, li, kx + 8 * lg)));
+                // kOff codes: the products start from -kOff X (the staged
+                // sums of tokens 4 lg .. 4 lg + 3), so the code offset
+                // cancels inside the product: D, not D + kOff X
+                qf4v c0 = zero;
+                if constexpr (kXsum) c0 = *reinterpret_cast<const qf4v *>(&xsum_s[cs * (kQChunk / kSub) + j][4 * lg]);
+                dv[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, b, c0, 0, 0, 0);
+                dv[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, b, dv[j], 0, 0, 0);
+                if (kPair) {
+                    dv2[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, b2, c0, 0, 0, 0);
+                    dv2[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, b2, dv2[j], 0, 0, 0);
                 }
             } else {
                 const s4v b = as_s4(r.step(j, sv[j]));
                 s4v b2 = b;
                 if (kPair) b2 = as_s4(r2.step(j, sv2[j]));
-#pragma unroll
-                for (int t = 0; t < TT; t++) {
-                    const s4v ah = as_s4(*reinterpret_cast<const uint2 *>(xs_at(0, 16 * t + li, kx + 4 * lg)));
-                    const s4v al = as_s4(*reinterpret_cast<const uint2 *>(xs_at(1, 16 * t + li, kx + 4 * lg)));
-                    dv[t][j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(ah, b, zero, 0, 0, 0);
-                    dv[t][j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(al, b, dv[t][j], 0, 0, 0);
-                    dv2[t][j] = zero;
-                    if (kPair) {
-                        dv2[t][j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(ah, b2, zero, 0, 0, 0);
-                        dv2[t][j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(al, b2, dv2[t][j], 0, 0, 0);
-                    }
+                const s4v ah = as_s4(*reinterpret_cast<const uint2 *>(xs_at(0, li, kx + 4 * lg)));
+                const s4v al = as_s4(*reinterpret_cast<const uint2 *>(xs_at(1, li, kx + 4 * lg)));
+                dv[j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(ah, b, zero, 0, 0, 0);
+                dv[j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(al, b, dv[j], 0, 0, 0);
+                if (kPair) {
+                    dv2[j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(ah, b2, zero, 0, 0, 0);
+                    dv2[j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(al, b2, dv2[j], 0, 0, 0);
                 }
             }
         }
 #pragma unroll
-        for (int j = j0; j < j0 + P; j++) {
+        for (int j = 0; j < S; j++) {
             const float s = sv[j] * live, s2 = sv2[j] * live;
 #pragma unroll
-            for (int t = 0; t < TT; t++)
-#pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    acc[t][q] = fmaf(s, dv[t][j][q], acc[t][q]);
-                    if (kPair) acc2[t][q] = fmaf(s2, dv2[t][j][q], acc2[t][q]);
-                }
-        }
+            for (int q = 0; q < 4; q++) {
+                acc[q] = fmaf(s, dv[j][q], acc[q]);
+                if (kPair) acc2[q] = fmaf(s2, dv2[j][q], acc2[q]);
+            }
         }
         if constexpr (kXsum) {
             // s D - min X, X the sub-block's activation sum: the minimum
@@ -634,15 +565,12 @@ __global__ void __launch_bounds__(256, OUT != OUT_SWIGLU ? 2 : 1) qgemm_kernel(Q
             r.min_coef(lg, c0, c1);
             c0 *= live, c1 *= live;
             if (kPair) r2.min_coef(lg, e0, e1), e0 *= live, e1 *= live;
-#pragma unroll
-            for (int t = 0; t < TT; t++) {
-                const float x0 = xsum_s[cs * 8 + lg][16 * t + li], x1 = xsum_s[cs * 8 + 4 + lg][16 * t + li];
-                acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(x0, c0, acc[t], 0, 0, 0);
-                acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(x1, c1, acc[t], 0, 0, 0);
-                if (kPair) {
-                    acc2[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(x0, e0, acc2[t], 0, 0, 0);
-                    acc2[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(x1, e1, acc2[t], 0, 0, 0);
-                }
+            const float x0 = xsum_s[cs * 8 + lg][li], x1 = xsum_s[cs * 8 + 4 + lg][li];
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(x0, c0, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(x1, c1, acc, 0, 0, 0);
+            if (kPair) {
+                acc2 = __builtin_amdgcn_mfma_f32_16x16x4f32(x0, e0, acc2, 0, 0, 0);
+                acc2 = __builtin_amdgcn_mfma_f32_16x16x4f32(x1, e1, acc2, 0, 0, 0);
             }
         }
     };
@@ -736,54 +664,51 @@ __global__ void __launch_bounds__(256, OUT != OUT_SWIGLU ? 2 : 1) qgemm_kernel(Q
         if constexpr (NRM) {
 #pragma unroll
             for (int o = 1; o < 16; o <<= 1) ssq += __shfl_xor(ssq, o, 64);
-            if (p.row_ss && blockIdx.x == 0 && part == 0 && tok_ok[0]) atomicAdd(p.row_ss + (m0 + tt), ssq);
+            if (p.row_ss && blockIdx.x == 0 && part == 0 && tok_ok) atomicAdd(p.row_ss + (m0 + tt), ssq);
         }
     };
-    // The results of group g: D[token 16 t + 4 lg + r][row li]; acc cleared after.
+    // The results of group g: D[token 4 lg + r][row li]; acc cleared after.
     auto epilogue = [&](int g) {
         const Seg sg = seg_of(g);
         const int nn = (g - sg.g0) * kQRows + 16 * wave + li;
 #pragma unroll
-        for (int t = 0; t < TT; t++) {
+        for (int r = 0; r < 4; r++) {
+            const int j = m0 + 4 * lg + r;  // token of result r
+            if (j >= M || nn >= sg.N) continue;
+            const int jrow = GROUPED ? ids[4 * lg + r] : j;
+            float *dst = sg.y ? sg.y + (size_t)jrow * sg.ldy + nn : nullptr;
+            const float v = acc[r];
+            if ((OUT == OUT_STORE || OUT == OUT_ADD) && p.ksplit > 1) {
+                atomicAdd(dst, v);  // partial sum of this workgroup's reduction range (STORE rows zeroed first)
+            } else if (OUT == OUT_STORE) {
+                *dst = v;
+            } else if (OUT == OUT_ADD) {
+                *dst = *dst + v;
+            } else if (OUT == OUT_SWIGLU) {
+                *dst = (v / (1.0f + expf(-v))) * acc2[r];
+            }
+        }
+        if (OUT == OUT_ARGMAX) {
+            // token 4 lg + r: the largest value over the 16 rows of lanes li, then the lowest row
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                const int j = m0 + 16 * t + 4 * lg + r;  // token of result r
-                if (j >= M || nn >= sg.N) continue;
-                const int jrow = GROUPED ? ids[16 * t + 4 * lg + r] : j;
-                float *dst = sg.y ? sg.y + (size_t)jrow * sg.ldy + nn : nullptr;
-                const float v = acc[t][r];
-                if ((OUT == OUT_STORE || OUT == OUT_ADD) && p.ksplit > 1) {
-                    atomicAdd(dst, v);  // partial sum of this workgroup's reduction range (STORE rows zeroed first)
-                } else if (OUT == OUT_STORE) {
-                    *dst = v;
-                } else if (OUT == OUT_ADD) {
-                    *dst = *dst + v;
-                } else if (OUT == OUT_SWIGLU) {
-                    *dst = (v / (1.0f + expf(-v))) * acc2[t][r];
-                }
-            }
-            if (OUT == OUT_ARGMAX) {
-                // token 4 lg + r: the largest value over the 16 rows of lanes li, then the lowest row
+                const int j = m0 + 4 * lg + r;
+                const float v = acc[r];
+                if (sg.y && j < M && nn < sg.N) sg.y[(size_t)j * sg.ldy + nn] = v;
+                unsigned long long key = (j < M && nn < sg.N)
+                                             ? ((unsigned long long)ordered_bits_q(v) << 32) |
+                                                   (unsigned long long)(0xFFFFFFFFu - (uint32_t)nn)
+                                             : 0ull;
 #pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    const int j = m0 + 16 * t + 4 * lg + r;
-                    const float v = acc[t][r];
-                    if (sg.y && j < M && nn < sg.N) sg.y[(size_t)j * sg.ldy + nn] = v;
-                    unsigned long long key = (j < M && nn < sg.N)
-                                                 ? ((unsigned long long)ordered_bits_q(v) << 32) |
-                                                       (unsigned long long)(0xFFFFFFFFu - (uint32_t)nn)
-                                                 : 0ull;
-#pragma unroll
-                    for (int o = 1; o < 16; o <<= 1) {
-                        const unsigned long long k2 = __shfl_xor(key, o, 64);
-                        key = k2 > key ? k2 : key;
-                    }
-                    if (li == 0 && key) atomicMax(p.argmax + j, key);
+                for (int o = 1; o < 16; o <<= 1) {
+                    const unsigned long long k2 = __shfl_xor(key, o, 64);
+                    key = k2 > key ? k2 : key;
                 }
+                if (li == 0 && key) atomicMax(p.argmax + j, key);
             }
-            acc[t] = qf4v{0.f, 0.f, 0.f, 0.f};
-            acc2[t] = qf4v{0.f, 0.f, 0.f, 0.f};
         }
+        acc = qf4v{0.f, 0.f, 0.f, 0.f};
+        acc2 = qf4v{0.f, 0.f, 0.f, 0.f};
     };
 
     if (nspan <= kStageChunks) {
@@ -819,14 +744,9 @@ __global__ void __launch_bounds__(256, OUT != OUT_SWIGLU ? 2 : 1) qgemm_kernel(Q
     // later stages wait for the ring's loads ahead of their activations.
     // kPre: the next stage's inputs are loaded into registers while this
     // stage computes, where the registers allow it without spills (the
-    // one-tile single products but Q3_K's, the split-input Q4_K / IQ4_XS
-    // ones and the grouped IQ4_XS pair); the last stage re-loads itself, so
-    // the loads stay unconditional.
-    // kPre1: the same for the one-chunk stages of the split-input Q8_0 kernel
-    constexpr bool kPre1 = XP && kStageChunks == 1 && F == Q8_0;
-    constexpr bool kPre = kStageChunks > 1 && (XP ? (F == Q4_K || F == IQ4_XS)
-                                               : GROUPED ? (kPair && F == IQ4_XS)
-                                                         : (!kPair && F != Q3_K));
+    // dense single products but Q3_K's and the grouped IQ4_XS pair); the last
+    // stage re-loads itself, so the loads stay unconditional.
+    constexpr bool kPre = kStageChunks > 1 && (GROUPED ? (kPair && F == IQ4_XS) : (!kPair && F != Q3_K));
     const int last_s0 = (nspan - 1) / kStageChunks * kStageChunks;
     auto prefetch = [&](int s0) {
         const int sn = min(s0, last_s0);
@@ -840,7 +760,7 @@ __global__ void __launch_bounds__(256, OUT != OUT_SWIGLU ? 2 : 1) qgemm_kernel(Q
         stage_store(nst);
         __syncthreads();
         fetch(0, 0, fa);
-        if constexpr (kPre || kPre1) prefetch(kStageChunks);
+        if constexpr (kPre) prefetch(kStageChunks);
         if constexpr (kStageChunks == 1) {
             fetch(1, 1, fb);  // chunk 0 only; the pairs below start at chunk 1
             compute(fa[0], fa[kMats - 1], 0, 1.f);
@@ -853,23 +773,19 @@ __global__ void __launch_bounds__(256, OUT != OUT_SWIGLU ? 2 : 1) qgemm_kernel(Q
         // and the ring slot of a chunk are its parity at compile time.
         for (int s0 = 1; s0 < nspan; s0 += 2) {
             __syncthreads();  // every wavefront is done with the previous stage
-            if constexpr (!kPre1) stage_load(kbeg + s0 * kQChunk, 1);
+            stage_load(kbeg + s0 * kQChunk, 1);
             stage_store(1);
             __syncthreads();
-            if constexpr (kPre1) prefetch(s0 + 1);
             fetch(0, s0 + 1, fa);
             compute(fb[0], fb[kMats - 1], 0, 1.f);
             // chunk s0 + 1 (past the range: a dead step, so the pairs stay whole)
             const bool more = s0 + 1 < nspan;
             __syncthreads();
-            if constexpr (kPre1) {
-                stage_store(more ? 1 : 0);  // (the loads land either way)
-            } else if (more) {
+            if (more) {
                 stage_load(kbeg + (s0 + 1) * kQChunk, 1);
                 stage_store(1);
             }
             __syncthreads();
-            if constexpr (kPre1) prefetch(s0 + 2);
             fetch(1, s0 + 2, fb);
             compute(fa[0], fa[kMats - 1], 0, more ? 1.f : 0.f);
         }
@@ -890,65 +806,39 @@ __global__ void __launch_bounds__(256, OUT != OUT_SWIGLU ? 2 : 1) qgemm_kernel(Q
 
 typedef void (*QGemmKernel)(QGemmParams);
 
-template <int F, bool G, int R, bool XP> static QGemmKernel pick_q(int out, bool nrm = false) {
-    if constexpr (!XP && !G && R == 2) {
-        if (nrm) return out == OUT_ADD ? qgemm_kernel<F, OUT_ADD, false, 2, false, true>
-                        : out == OUT_STORE ? qgemm_kernel<F, OUT_STORE, false, 2, false, true>
+// ring depth 2: two workgroups per CU leave stages of two chunks
+template <int F, bool G> static QGemmKernel pick_q(int out, bool nrm = false) {
+    if constexpr (!G) {
+        if (nrm) return out == OUT_ADD ? qgemm_kernel<F, OUT_ADD, false, 2, true>
+                        : out == OUT_STORE ? qgemm_kernel<F, OUT_STORE, false, 2, true>
                                            : nullptr;
-    } else {
-        if (nrm) return nullptr;
+        if (out == OUT_ADD) return qgemm_kernel<F, OUT_ADD, false, 2>;
+        if (out == OUT_ARGMAX) return qgemm_kernel<F, OUT_ARGMAX, false, 2>;
+    } else if (nrm) {
+        return nullptr;
     }
-    if constexpr (XP) {
-        // split inputs, two token tiles: the dense stores and adds of the batched passes
-        if constexpr (G || R != 2)
-            return nullptr;
-        else
-            return out == OUT_STORE ? qgemm_kernel<F, OUT_STORE, G, R, XP>
-                   : out == OUT_ADD ? qgemm_kernel<F, OUT_ADD, G, R, XP>
-                                    : nullptr;
-    } else if constexpr (R != 2) {
-        return nullptr;  // ring depth 2: stages may hold two chunks
-    } else {
-        switch (out) {
-        case OUT_STORE: return qgemm_kernel<F, OUT_STORE, G, R, XP>;
-        case OUT_SWIGLU:
-            if constexpr (R == 2) return qgemm_kernel<F, OUT_SWIGLU, G, R, XP>;  // deeper rings spill
-            return nullptr;
-        case OUT_ADD:
-            if constexpr (G) return nullptr;
-            else return qgemm_kernel<F, OUT_ADD, G, R, XP>;
-        case OUT_ARGMAX:
-            if constexpr (G) return nullptr;
-            else return qgemm_kernel<F, OUT_ARGMAX, G, R, XP>;
-        default: return nullptr;
-        }
-    }
+    return out == OUT_STORE ? qgemm_kernel<F, OUT_STORE, G, 2> : out == OUT_SWIGLU ? qgemm_kernel<F, OUT_SWIGLU, G, 2> : nullptr;
 }
-
-// ring depth: 4 chunks, or 2 for the two matrices of SWIGLU (the same bytes in
-// flight), for reduction ranges of two chunks, for two token tiles (the
-// products' registers) and for the grouped kernels (stages of two chunks)
-template <bool G, bool XP> static QGemmKernel pick_qf(int fmt, int out, int K, bool nrm = false) {
-    (void)K;
-    switch (fmt) {  // every kernel at depth 2 (two workgroups per CU leave stages of two chunks)
-    case Q4_K: return pick_q<Q4_K, G, 2, XP>(out, nrm);
-    case Q6_K: return pick_q<Q6_K, G, 2, XP>(out, nrm);
-    case Q8_0: return pick_q<Q8_0, G, 2, XP>(out, nrm);
-    case IQ4_XS: return pick_q<IQ4_XS, G, 2, XP>(out, nrm);
-    case Q3_K: return pick_q<Q3_K, G, 2, XP>(out, nrm);
+template <bool G> static QGemmKernel pick_qf(int fmt, int out, bool nrm = false) {
+    switch (fmt) {
+    case Q4_K: return pick_q<Q4_K, G>(out, nrm);
+    case Q6_K: return pick_q<Q6_K, G>(out, nrm);
+    case Q8_0: return pick_q<Q8_0, G>(out, nrm);
+    case IQ4_XS: return pick_q<IQ4_XS, G>(out, nrm);
+    case Q3_K: return pick_q<Q3_K, G>(out, nrm);
     default: return nullptr;
     }
 }
 
 // The chunk windows assume a 16-byte aligned matrix (and expert slices) whose
 // row stride keeps chunk addresses within the format's offsets below 16.
-template <bool P, int TT = 1, int OCC = 1> static int stage_chunks_of(int fmt) {
+template <bool P, int OCC = 1> static int stage_chunks_of(int fmt) {
     switch (fmt) {
-    case Q4_K: return QGeom<Q4_K, P, TT, OCC>::kStageChunks;
-    case Q8_0: return QGeom<Q8_0, P, TT, OCC>::kStageChunks;
-    case IQ4_XS: return QGeom<IQ4_XS, P, TT, OCC>::kStageChunks;
-    case Q6_K: return QGeom<Q6_K, P, TT, OCC>::kStageChunks;
-    case Q3_K: return QGeom<Q3_K, P, TT, OCC>::kStageChunks;
+    case Q4_K: return QGeom<Q4_K, P, OCC>::kStageChunks;
+    case Q8_0: return QGeom<Q8_0, P, OCC>::kStageChunks;
+    case IQ4_XS: return QGeom<IQ4_XS, P, OCC>::kStageChunks;
+    case Q6_K: return QGeom<Q6_K, P, OCC>::kStageChunks;
+    case Q3_K: return QGeom<Q3_K, P, OCC>::kStageChunks;
     default: return 0;
     }
 }
@@ -999,7 +889,7 @@ static double qgemm_stage_weight() {
 
 hipError_t launch_qgemm_multi(int fmt, int nseg, const uint8_t *const *w, float *const *y, const int *ldy,
                               const int *N, const uint8_t *w2, uint64_t stride, const float *x, int ldx, int M, int K,
-                              int out, unsigned long long *argmax, hipStream_t s, int max_split, const XPlanes *xp,
+                              int out, unsigned long long *argmax, hipStream_t s, int max_split,
                               const RowNorm *rn) {
     if (nseg < 1 || nseg > 3 || M < 1 || ldx % 4 || (nseg > 1 && (out == OUT_SWIGLU || out == OUT_ARGMAX)))
         return hipErrorInvalidValue;
@@ -1019,15 +909,9 @@ hipError_t launch_qgemm_multi(int fmt, int nseg, const uint8_t *const *w, float 
     }
     p.groups = groups;
     p.nseg = nseg;
-    // split inputs (more than one token tile): the XP kernels, two token tiles per workgroup
-    const bool use_xp = !rn && xp && xp->hi && xp->lo && xp->sum && xp->ld % 32 == 0 && K <= xp->ld && M > 16 &&
-                        (out == OUT_STORE || out == OUT_ADD);
-    const int TT = use_xp ? 2 : 1;
-    const int tiles = (M + 16 * TT - 1) / (16 * TT), chunks = K / kQChunk;
+    const int tiles = (M + 15) / 16, chunks = K / kQChunk;
     const int target = qgemm_target_wgs();
-    int stage = use_xp                ? stage_chunks_of<false, 2, 2>(fmt)
-                : out == OUT_SWIGLU ? stage_chunks_of<true>(fmt)
-                                    : stage_chunks_of<false, 1, 2>(fmt);
+    int stage = out == OUT_SWIGLU ? stage_chunks_of<true>(fmt) : stage_chunks_of<false, 2>(fmt);
     if (rn && stage > kNrmStage / kQChunk) stage = kNrmStage / kQChunk;  // the NRM kernels' stages
     // Reduction split ks (a power of two; results added atomically, plain
     // stores and adds only) and workgroups per split pg, each taking every
@@ -1053,13 +937,12 @@ hipError_t launch_qgemm_multi(int fmt, int nseg, const uint8_t *const *w, float 
             while (groups * tiles * ks * 2 <= target && chunks % (ks * 2) == 0 && ks * 2 <= max_split) ks *= 2;
     }
     p.ksplit = ks;
-    QGemmKernel k = use_xp ? pick_qf<false, true>(fmt, out, K / ks) : pick_qf<false, false>(fmt, out, K / ks, rn);
+    QGemmKernel k = pick_qf<false>(fmt, out, rn);
     if (!k) return hipErrorInvalidValue;
     if (rn) {
         p.norm_w = rn->w;
         p.row_ss = rn->ss;  // none: another launch over the same rows adds the sums
     }
-    if (use_xp) p.xh = xp->hi, p.xl = xp->lo, p.xsum = xp->sum, p.ldxs = xp->ld;
     if (ks > 1 && out == OUT_STORE) {
         for (int i = 0; i < nseg; i++) {
             hipLaunchKernelGGL(zero_rows_kernel, dim3((M * N[i] + 255) / 256), dim3(256), 0, s, y[i], ldy[i], M, N[i]);
@@ -1073,8 +956,8 @@ hipError_t launch_qgemm_multi(int fmt, int nseg, const uint8_t *const *w, float 
 
 hipError_t launch_qgemm(int fmt, const uint8_t *w, const uint8_t *w2, uint64_t stride, const float *x, int ldx,
                         float *y, int ldy, int M, int N, int K, int out, unsigned long long *argmax, hipStream_t s,
-                        int max_split, const XPlanes *xp) {
-    return launch_qgemm_multi(fmt, 1, &w, &y, &ldy, &N, w2, stride, x, ldx, M, K, out, argmax, s, max_split, xp);
+                        int max_split) {
+    return launch_qgemm_multi(fmt, 1, &w, &y, &ldy, &N, w2, stride, x, ldx, M, K, out, argmax, s, max_split);
 }
 
 hipError_t launch_qgemm_grouped(int fmt, const uint8_t *w, const uint8_t *w2, uint64_t stride,
@@ -1083,7 +966,7 @@ hipError_t launch_qgemm_grouped(int fmt, const uint8_t *w, const uint8_t *w2, ui
                                 hipStream_t s) {
     if (N < 1 || !qgemm_supported(fmt, K, w, w2, stride, expert_stride) || ldx % 4 || max_tiles < 1 || x_div < 1)
         return hipErrorInvalidValue;
-    QGemmKernel k = pick_qf<true, false>(fmt, out, K);
+    QGemmKernel k = pick_qf<true>(fmt, out);
     if (!k) return hipErrorInvalidValue;
     QGemmParams p{w, w2, stride, x, y, 16, N, K, ldx, ldy, nullptr, tiles, list, ntiles, x_div, expert_stride, 1};
     p.groups = (N + kQRows - 1) / kQRows;
@@ -1091,7 +974,7 @@ hipError_t launch_qgemm_grouped(int fmt, const uint8_t *w, const uint8_t *w2, ui
     // A one-stage reduction lets a workgroup take several row groups of its
     // token tile against one staging: about four workgroups per CU at the
     // largest tile count (the launch's bound; unused tiles exit at once).
-    const int stage = out == OUT_SWIGLU ? stage_chunks_of<true, 1, 2>(fmt) : stage_chunks_of<false, 1, 3>(fmt);
+    const int stage = out == OUT_SWIGLU ? stage_chunks_of<true, 2>(fmt) : stage_chunks_of<false, 3>(fmt);
     int pg = p.groups;
     if (K / kQChunk <= stage) {
         pg = 4 * qgemm_target_wgs() / max_tiles;

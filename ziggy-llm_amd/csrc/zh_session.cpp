@@ -16,6 +16,7 @@
 // device memory, so the same graph replays every step.
 #include <algorithm>
 #include <chrono>
+#include <initializer_list>
 #include <new>
 #include <vector>
 
@@ -89,7 +90,7 @@ struct ZiggyHipSession {
     // batched verify (allocated on first use): [kVerifyMax] rows each
     float *b_hidden = nullptr, *b_normed = nullptr, *b_q = nullptr, *b_k = nullptr, *b_v = nullptr;
     float *b_attn = nullptr, *b_act = nullptr, *b_up = nullptr, *b_logits = nullptr;
-    float *b_ss = nullptr;  // verify: the deferred norms' row sums of squares, [2][kPassMax]
+    float *b_ss = nullptr;  // verify: the deferred norms' row sums of squares, [2][kPassBase]
     // output shortlist (allocated on first use): packed keys, entries
     unsigned long long *sl_keys = nullptr;
     uint32_t *sl_entries = nullptr;
@@ -98,7 +99,12 @@ struct ZiggyHipSession {
     // multi-query attention of a verify pass: partials and arrival counters
     // of head_count_kv * query-group slots
     float *b_part_o = nullptr, *b_part_ml = nullptr;
-    zh::XPlanes xp{};  // the o and down products' inputs, split once per pass
+    // prompt passes: rows of the pass buffers above (pass_rows), the products' inputs as planes
+    // and the workspace of their split reductions
+    uint32_t pass_rows = 0;
+    std::vector<void *> pass_allocs;
+    zh::HPlanes hp{};
+    float *pg_part = nullptr;
     unsigned *b_counters = nullptr;
     uint32_t position = 0;
     // the token whose K/V rows sit at each position below `position`, while
@@ -415,6 +421,7 @@ void free_session(ZiggyHipSession *s) {
     }
     if (s->graph) hipGraphExecDestroy(s->graph);
     for (void *p : s->allocs) hipFree(p);
+    for (void *p : s->pass_allocs) hipFree(p);
     if (s->st_host) hipHostFree(s->st_host);
     delete s;
 }
@@ -888,12 +895,16 @@ int ziggy_hip_session_step_shortlist(ZiggyHipSession *s, uint32_t token, uint32_
 
 }  // extern "C"
 
-static hipError_t pass_alloc(ZiggyHipSession *s);
+static hipError_t pass_alloc(ZiggyHipSession *s, uint32_t rows);
 static hipError_t pass_enqueue(ZiggyHipSession *s, const uint32_t *tokens, int M, int pos, bool output,
                                hipStream_t st);
-constexpr uint32_t kPrefillMax = 256;  // prompt rows per batched pass at most (the pass buffers' row count)
-// prompt rows per batched pass (ZIGGY_HIP_PREFILL_CHUNK, 16 .. 256; a tuning knob): the whole
-// buffer by default (4096 tokens: 725 ms in passes of 64, 635 in 128, 613 in 256)
+// Prompt rows per batched pass at most: a 4096-row product of a 4096-row matrix is 256 tiles of
+// 256 x 256, one per CU (Llama-8B-shaped 4096-token prompt, 4 layers: 46.6 ms in passes of 256).
+constexpr uint32_t kPrefillMax = 4096;
+// Passes of models with a matrix that the prompt products don't take (pgemm_supported), and the
+// attention launches of a pass, whose split partials are sized for this many queries.
+constexpr uint32_t kPassBase = 256;
+// prompt rows per batched pass (ZIGGY_HIP_PREFILL_CHUNK, 16 .. 4096; a tuning knob)
 static uint32_t prefill_chunk() {
     static const uint32_t v = [] {
         const char *e = getenv("ZIGGY_HIP_PREFILL_CHUNK");
@@ -901,6 +912,16 @@ static uint32_t prefill_chunk() {
         return (uint32_t)(c < 16 ? 16 : c > (int)kPrefillMax ? (int)kPrefillMax : c);
     }();
     return v;
+}
+static bool pg_ok(const DT &d) { return pgemm_supported((int)d.type, (int)d.cols, d.p, d.stride); }
+// whether every product of a prompt pass runs from planes
+static bool pg_all(const ZiggyHipSession *s) {
+    for (const LayerW &L : s->layers) {
+        for (const DT *d : {&L.q, &L.k, &L.v, &L.o, &L.gate, &L.up, &L.down})
+            if (!pg_ok(*d)) return false;
+        if (L.gate.type != L.up.type || L.gate.stride != L.up.stride) return false;
+    }
+    return true;
 }
 
 // Prompt rows go through batched passes on the matrix cores unless the head
@@ -965,7 +986,7 @@ int ziggy_hip_session_generate(ZiggyHipSession *s, const uint32_t *prompt, uint3
     // the prompt token by token (runPrompt, model/loader.zig:1016-1036)
     const bool batched = prompt_len > 1 && prefill_batched(s);
     const uint32_t n_batched = batched ? prompt_len - 1 : 0;
-    if (batched) ZH_TRY(pass_alloc(s), "prefill buffers");
+    if (batched) ZH_TRY(pass_alloc(s, n_batched), "prefill buffers");
     StepState *h = s->st_host;
     memset(h, 0, sizeof(*h));
     h->mode = 1;
@@ -976,7 +997,7 @@ int ziggy_hip_session_generate(ZiggyHipSession *s, const uint32_t *prompt, uint3
     ZH_TRY(hipMemcpyAsync(s->st, h, sizeof(StepState), hipMemcpyHostToDevice, st), "step state");
     ZH_TRY(hipStreamSynchronize(st), "generate setup");
     const uint64_t tp0 = now_ns();
-    const uint32_t chunk = prefill_chunk();
+    const uint32_t chunk = std::min(prefill_chunk(), s->pass_rows);
     for (uint32_t off = 0; off < n_batched; off += chunk) {
         const uint32_t m = std::min(chunk, n_batched - off);
         ZH_TRY(pass_enqueue(s, s->prompt + off, (int)m, (int)(s->position + off), false, st), "prefill pass");
@@ -1016,53 +1037,77 @@ int ziggy_hip_session_generate(ZiggyHipSession *s, const uint32_t *prompt, uint3
 // ---- speculative verify: a batch of tokens in one pass ----
 
 constexpr uint32_t kVerifyMax = 16;  // tokens of one verify pass (one MFMA token tile)
-constexpr uint32_t kPassMax = kPrefillMax;  // token rows of one batched pass
-static_assert(kPassMax >= kVerifyMax, "a verify pass fits the pass buffers");
+static_assert(kPassBase >= kVerifyMax, "a verify pass fits the pass buffers");
+constexpr size_t kPgPart = 16u << 20;  // floats of the split reductions' workspace
 
-// Row buffers of the batched passes (verify, prompt chunks), allocated on first use.
-static hipError_t pass_alloc(ZiggyHipSession *s) {
-    if (s->b_hidden) return hipSuccess;
+// Row buffers of the batched passes (verify, prompt chunks) for at least `rows` rows: kPassBase at
+// first; more (up to kPrefillMax) for a longer prompt where every product runs from planes, or as
+// many as memory allows.
+static hipError_t pass_alloc(ZiggyHipSession *s, uint32_t rows) {
+    rows = std::min((rows + kPassBase - 1) / kPassBase * kPassBase, prefill_chunk());
+    if (rows < kPassBase || !pg_all(s)) rows = kPassBase;
+    if (rows <= s->pass_rows) return hipSuccess;
     const size_t H = s->md.embedding_length, F = s->md.feed_forward_length, Q = (size_t)s->q_size,
-                 KV = (size_t)s->kv_size, M = kPassMax;
-    struct {
-        void **p;
-        size_t bytes;
-    } reqs[] = {{(void **)&s->b_hidden, M * H * 4}, {(void **)&s->b_normed, M * H * 4}, {(void **)&s->b_q, M * Q * 4},
-                {(void **)&s->b_k, M * KV * 4},      {(void **)&s->b_v, M * KV * 4},      {(void **)&s->b_attn, M * Q * 4},
-                {(void **)&s->b_act, M * F * 4},     {(void **)&s->b_up, M * F * 4},      {(void **)&s->b_tokens, M * 4},
-                {(void **)&s->b_argmax, M * 8},     {(void **)&s->b_logits, kVerifyMax * s->md.vocab_size * 4},
-                {(void **)&s->b_ss, 2 * M * 4}};
-    for (auto &r : reqs) {
-        hipError_t e = hipMalloc(r.p, r.bytes);
-        if (e != hipSuccess) return e;
-        s->allocs.push_back(*r.p);
+                 KV = (size_t)s->kv_size, B = kPassBase;
+    // buffers whose size doesn't follow the rows, once
+    if (!s->b_tokens) {
+        struct {
+            void **p;
+            size_t bytes;
+        } reqs[] = {{(void **)&s->b_normed, B * H * 4}, {(void **)&s->b_up, B * F * 4},
+                    {(void **)&s->b_argmax, B * 8},     {(void **)&s->b_logits, kVerifyMax * s->md.vocab_size * 4},
+                    {(void **)&s->b_ss, 2 * B * 4},     {(void **)&s->pg_part, kPgPart * 4},
+                    {(void **)&s->b_tokens, B * 4}};
+        for (auto &r : reqs) {
+            hipError_t e = hipMalloc(r.p, r.bytes);
+            if (e != hipSuccess) return e;
+            s->allocs.push_back(*r.p);
+        }
+        if (attention_multi_supported((int)s->md.head_dim)) {
+            const size_t slots = (size_t)s->md.head_count_kv *
+                                 attention_query_groups((int)s->md.head_count, (int)s->md.head_count_kv, (int)B);
+            const size_t po = slots * s->max_splits * kMultiHeads * s->md.head_dim,
+                         pml = slots * s->max_splits * kMultiHeads * 2;
+            hipError_t e = hipMalloc((void **)&s->b_part_o, (po + pml) * 4);
+            if (e != hipSuccess) return e;
+            s->allocs.push_back(s->b_part_o);
+            s->b_part_ml = s->b_part_o + po;
+            e = hipMalloc((void **)&s->b_counters, slots * sizeof(unsigned));
+            if (e != hipSuccess) return e;
+            s->allocs.push_back(s->b_counters);
+            e = hipMemsetAsync(s->b_counters, 0, slots * sizeof(unsigned), s->ctx->stream);  // the merge resets them
+            if (e != hipSuccess) return e;
+        }
     }
-    {
-        const size_t ld = (std::max(std::max(Q, F), H) + 31) / 32 * 32;
-        uint8_t *base = nullptr;
-        hipError_t e = hipMalloc((void **)&base, M * ld * 4 + M * (ld / 32) * 4);
-        if (e != hipSuccess) return e;
-        s->allocs.push_back(base);
-        s->xp.hi = reinterpret_cast<uint16_t *>(base);
-        s->xp.lo = s->xp.hi + M * ld;
-        s->xp.sum = reinterpret_cast<float *>(s->xp.lo + M * ld);
-        s->xp.ld = (int)ld;
+    // the row buffers, again for more rows (hipFree waits for the passes that used them)
+    for (void *p : s->pass_allocs) hipFree(p);
+    s->pass_allocs.clear();
+    s->pass_rows = 0;
+    const size_t W = std::max(std::max(Q, F), H), nblk = W / 256 + 1;
+    for (;;) {
+        const size_t M = rows;
+        struct {
+            void **p;
+            size_t bytes;
+        } reqs[] = {{(void **)&s->b_hidden, M * H * 4}, {(void **)&s->b_q, M * Q * 4},
+                    {(void **)&s->b_k, M * KV * 4},     {(void **)&s->b_v, M * KV * 4},
+                    {(void **)&s->b_attn, M * Q * 4},   {(void **)&s->b_act, M * F * 4},
+                    {(void **)&s->hp.x, M * nblk * 256 * 4}, {(void **)&s->hp.xs, M * nblk * 32},
+                    {(void **)&s->hp.scale, M * 4}};
+        hipError_t e = hipSuccess;
+        for (auto &r : reqs) {
+            e = hipMalloc(r.p, r.bytes);
+            if (e != hipSuccess) break;
+            s->pass_allocs.push_back(*r.p);
+        }
+        if (e == hipSuccess) break;
+        (void)hipGetLastError();
+        for (void *p : s->pass_allocs) hipFree(p);
+        s->pass_allocs.clear();
+        if (rows == kPassBase) return e;
+        rows = std::max(kPassBase, rows / 2 / kPassBase * kPassBase);
     }
-    if (attention_multi_supported((int)s->md.head_dim)) {
-        const size_t slots = (size_t)s->md.head_count_kv *
-                             attention_query_groups((int)s->md.head_count, (int)s->md.head_count_kv, (int)M);
-        const size_t po = slots * s->max_splits * kMultiHeads * s->md.head_dim,
-                     pml = slots * s->max_splits * kMultiHeads * 2;
-        hipError_t e = hipMalloc((void **)&s->b_part_o, (po + pml) * 4);
-        if (e != hipSuccess) return e;
-        s->allocs.push_back(s->b_part_o);
-        s->b_part_ml = s->b_part_o + po;
-        e = hipMalloc((void **)&s->b_counters, slots * sizeof(unsigned));
-        if (e != hipSuccess) return e;
-        s->allocs.push_back(s->b_counters);
-        e = hipMemsetAsync(s->b_counters, 0, slots * sizeof(unsigned), s->ctx->stream);  // the merge resets them
-        if (e != hipSuccess) return e;
-    }
+    s->pass_rows = rows;
     return hipSuccess;
 }
 
@@ -1103,24 +1148,34 @@ static hipError_t pass_enqueue(ZiggyHipSession *s, const uint32_t *tokens, int M
         return n == 1 || n == 2 || n == 4 || n == 8 || n == 16 ? n : 16;
     }();
     const int split_add = det ? 1 : vsplit, split_clear = det ? 2 : vsplit;
-    auto gemm = [&](const DT &w, const DT *w2, const float *x, int ldx, float *y, int ldy, int out,
-                    const XPlanes *xp = nullptr) {
+    auto gemm = [&](const DT &w, const DT *w2, const float *x, int ldx, float *y, int ldy, int out) {
         if (e != hipSuccess) return;
         e = launch_gemm(w.type, w.p, w2 ? w2->p : nullptr, w.stride, x, ldx, y, ldy, M, (int)w.rows, (int)w.cols,
-                        out, s->b_argmax, st, false, out == OUT_ADD ? split_add : split_clear, xp);
+                        out, s->b_argmax, st, false, out == OUT_ADD ? split_add : split_clear);
     };
-    // Prompt passes of more than one token tile give the products their
-    // inputs as pieces split once here: the products then take two token
-    // tiles per workgroup, and no workgroup splits the rows again.  (A verify
-    // pass, one token tile, lets the products split their own.)
-    const bool split_in = det && M > 16 && H % 32 == 0, split_o = det && M > 16 && Q % 32 == 0,
-               split_down = det && M > 16 && F % 32 == 0;
+    // Prompt passes of more than 16 rows (one token tile of the products above): every product
+    // that takes them runs from planes, split once per input (zh_pgemm.hip).
+    const bool planes = det && M > 16;
+    auto pgemm = [&](int n, const DT *const *d, const DT *w2, float *const *ys, const int *lds, int out) {
+        if (e != hipSuccess) return;
+        const uint8_t *ws[3];
+        int Ns[3];
+        for (int i = 0; i < n; i++) ws[i] = d[i]->p, Ns[i] = (int)d[i]->rows;
+        e = launch_pgemm((int)d[0]->type, n, ws, w2 ? w2->p : nullptr, ys, lds, Ns, d[0]->stride, s->hp, M,
+                         (int)d[0]->cols, out, s->pg_part, kPgPart, st);
+    };
+    // onto the residual: from the rows' planes where the product takes them
+    auto add_product = [&](const DT &w, const float *x, int ldx, float *y, int ldy) {
+        if (!planes || !pg_ok(w)) return gemm(w, nullptr, x, ldx, y, ldy, OUT_ADD);
+        if (e == hipSuccess) e = launch_row_planes(x, ldx, M, (int)w.cols, s->hp, st);
+        const DT *d[1] = {&w};
+        pgemm(1, d, nullptr, &y, &ldy, OUT_ADD);
+    };
     // products of the normed rows that accumulate (OUT_ADD) onto cleared
     // outputs, or store them (no reduction split): one launch for the
     // matrices that share a format and row size
     auto multi3 = [&](const DT &a, float *ya, int lda, const DT &b, float *yb, int ldb, const DT *c, float *yc,
-                      int ldc, const XPlanes *xp, bool store = false, const float *xin = nullptr,
-                      const RowNorm *rn = nullptr) {
+                      int ldc, bool store = false, const float *xin = nullptr, const RowNorm *rn = nullptr) {
         if (e != hipSuccess) return;
         if (!xin) xin = s->b_normed;
         const DT *d[3] = {&a, &b, c};
@@ -1131,16 +1186,30 @@ static hipError_t pass_enqueue(ZiggyHipSession *s, const uint32_t *tokens, int M
         while (i < n && e == hipSuccess) {
             int j = i + 1;  // a run of matrices of one type and row size
             while (j < n && d[j]->type == d[i]->type && d[j]->stride == d[i]->stride && d[j]->cols == d[i]->cols) j++;
+            if (planes && pg_ok(*d[i])) {
+                pgemm(j - i, d + i, nullptr, ys + i, lds + i, OUT_STORE);
+                i = j;
+                continue;
+            }
             const uint8_t *ws[3];
             int Ns[3];
             for (int k = i; k < j; k++) ws[k - i] = d[k]->p, Ns[k - i] = (int)d[k]->rows;
             // the deferred norm's row sums once: with the first run of matrices
             const RowNorm rn_i = rn ? RowNorm{rn->w, i == 0 ? rn->ss : nullptr} : RowNorm{};
             e = launch_gemm_multi(d[i]->type, j - i, ws, ys + i, lds + i, Ns, d[i]->stride, xin, H, M,
-                                  (int)d[i]->cols, store ? OUT_STORE : OUT_ADD, st, store ? 1 : split_clear, xp,
+                                  (int)d[i]->cols, store ? OUT_STORE : OUT_ADD, st, store ? 1 : split_clear,
                                   rn ? &rn_i : nullptr);
             i = j;
         }
+    };
+    // The hidden rows' norm into planes where one of the products takes them (and into b_normed for
+    // the others); false: none does.
+    auto norm_planes = [&](const float *w, std::initializer_list<const DT *> mats) {
+        bool any = false, all = true;
+        for (const DT *d : mats) (pg_ok(*d) ? any : all) = pg_ok(*d);
+        if (!planes || !any || e != hipSuccess) return false;
+        e = launch_norm_planes(s->b_hidden, w, all ? nullptr : s->b_normed, M, H, eps, s->hp, st);
+        return true;
     };
     // Verify passes defer the RMSNorms (RowNorm): the q/k/v and gate/up
     // products take hidden * norm weights and add each row's sum of squares
@@ -1155,7 +1224,7 @@ static hipError_t pass_enqueue(ZiggyHipSession *s, const uint32_t *tokens, int M
         for (const DT *d : {&L.q, &L.k, &L.v, &L.gate, &L.up})
             dn = dn && gemm_rownorm_supported(d->type, (int)d->cols, d->p, d->stride);
     }
-    float *ss_attn = s->b_ss, *ss_ffn = s->b_ss ? s->b_ss + kPassMax : nullptr;
+    float *ss_attn = s->b_ss, *ss_ffn = s->b_ss ? s->b_ss + kPassBase : nullptr;
     const ZeroSpans clear_qkv{{s->b_q, s->b_k, s->b_v, ss_attn}, {(size_t)M * Q, (size_t)M * KV, (size_t)M * KV, (size_t)M}};
     const ZeroSpans clear_ffn{{s->b_act, s->b_up, ss_ffn, nullptr}, {(size_t)M * F, (size_t)M * F, (size_t)M, 0}};
     if (dn && e == hipSuccess) e = launch_zero_spans(clear_qkv, st);
@@ -1163,13 +1232,15 @@ static hipError_t pass_enqueue(ZiggyHipSession *s, const uint32_t *tokens, int M
         const LayerW &L = s->layers[l];
         if (dn) {
             const RowNorm rn{(const float *)L.attn_norm.p, ss_attn};
-            multi3(L.q, s->b_q, Q, L.k, s->b_k, KV, &L.v, s->b_v, KV, nullptr, false, s->b_hidden, &rn);
+            multi3(L.q, s->b_q, Q, L.k, s->b_k, KV, &L.v, s->b_v, KV, false, s->b_hidden, &rn);
+        } else if (norm_planes((const float *)L.attn_norm.p, {&L.q, &L.k, &L.v})) {
+            multi3(L.q, s->b_q, Q, L.k, s->b_k, KV, &L.v, s->b_v, KV, true);
         } else {
             // the norm clears the q/k/v rows, which the products then accumulate onto
-            e = launch_rms_norm_rows(s->b_hidden, (const float *)L.attn_norm.p, s->b_normed, M, H, eps, st, s->b_q,
-                                     (size_t)M * Q, s->b_k, (size_t)M * KV, s->b_v, (size_t)M * KV,
-                                     split_in ? &s->xp : nullptr);
-            multi3(L.q, s->b_q, Q, L.k, s->b_k, KV, &L.v, s->b_v, KV, split_in ? &s->xp : nullptr);
+            if (e == hipSuccess)
+                e = launch_rms_norm_rows(s->b_hidden, (const float *)L.attn_norm.p, s->b_normed, M, H, eps, st, s->b_q,
+                                         (size_t)M * Q, s->b_k, (size_t)M * KV, s->b_v, (size_t)M * KV);
+            multi3(L.q, s->b_q, Q, L.k, s->b_k, KV, &L.v, s->b_v, KV);
         }
         const size_t layer_base = kv_layer_base(s, l);
         if (s->b_counters && e == hipSuccess) {
@@ -1211,7 +1282,14 @@ static hipError_t pass_enqueue(ZiggyHipSession *s, const uint32_t *tokens, int M
             a.window_start = 0;
             a.scale = 1.0f / sqrtf((float)md.head_dim);
             a.max_splits = s->max_splits;
-            if (e == hipSuccess) e = launch_attention(a, st);
+            for (int m = 0; m < M && e == hipSuccess; m += (int)kPassBase) {
+                AttnParams c = a;
+                c.q = s->b_q + (size_t)m * Q;
+                c.out = s->b_attn + (size_t)m * Q;
+                c.position = pos + m;
+                c.n_query = std::min(M - m, (int)kPassBase);
+                e = launch_attention(c, st);
+            }
         }
         // token by token where the multi-query kernel does not serve the shape (head_dim 256, the
         // vector kernel): never with the polled merge, which needs the matrix-core kernel too
@@ -1249,32 +1327,34 @@ static hipError_t pass_enqueue(ZiggyHipSession *s, const uint32_t *tokens, int M
             a.ctx = (int)md.context_length;
             e = launch_attention(a, st);
         }
-        if (split_o && e == hipSuccess) e = launch_split_rows(s->b_attn, Q, M, Q, s->xp, st);
-        gemm(L.o, nullptr, s->b_attn, Q, s->b_hidden, H, OUT_ADD, split_o ? &s->xp : nullptr);
-        bool down_split = false;
+        add_product(L.o, s->b_attn, Q, s->b_hidden, H);
         if (dn) {
             const RowNorm rn{(const float *)L.ffn_norm.p, ss_ffn};
-            multi3(L.gate, s->b_act, F, L.up, s->b_up, F, nullptr, nullptr, 0, nullptr, false, s->b_hidden, &rn);
+            multi3(L.gate, s->b_act, F, L.up, s->b_up, F, nullptr, nullptr, 0, false, s->b_hidden, &rn);
             if (e == hipSuccess) e = launch_silu_mul_rows(s->b_act, s->b_up, M, F, RowScale{ss_ffn, H, eps}, clear_qkv, st);
-        } else if (fused_swiglu && L.gate.type == L.up.type) {
+        } else if (fused_swiglu && !planes && L.gate.type == L.up.type) {
             if (e == hipSuccess)
                 e = launch_rms_norm_rows(s->b_hidden, (const float *)L.ffn_norm.p, s->b_normed, M, H, eps, st);
             gemm(L.gate, &L.up, s->b_normed, H, s->b_act, F, OUT_SWIGLU);
+        } else if (planes && pg_ok(L.gate) && pg_ok(L.up) && L.gate.type == L.up.type && L.gate.stride == L.up.stride) {
+            // both products of a row and SiLU(gate) * up in one launch
+            norm_planes((const float *)L.ffn_norm.p, {&L.gate, &L.up});
+            const DT *d[1] = {&L.gate};
+            float *ys[1] = {s->b_act};
+            const int lds[1] = {F};
+            pgemm(1, d, &L.up, ys, lds, OUT_SWIGLU);
         } else {
             // gate and up (prompt chunks: stores; verify passes: onto rows
             // the norm clears, each product may split its reduction), then
             // SiLU(gate) * up
-            if (e == hipSuccess)
+            if (!norm_planes((const float *)L.ffn_norm.p, {&L.gate, &L.up}) && e == hipSuccess)
                 e = launch_rms_norm_rows(s->b_hidden, (const float *)L.ffn_norm.p, s->b_normed, M, H, eps, st,
                                          det ? nullptr : s->b_act, det ? 0 : (size_t)M * F, det ? nullptr : s->b_up,
-                                         det ? 0 : (size_t)M * F, nullptr, 0, split_in ? &s->xp : nullptr);
-            multi3(L.gate, s->b_act, F, L.up, s->b_up, F, nullptr, nullptr, 0, split_in ? &s->xp : nullptr, det);
-            down_split = split_down;
-            if (e == hipSuccess)
-                e = down_split ? launch_silu_mul_split(s->b_act, s->b_up, M, F, s->xp, st)
-                               : launch_silu_mul(s->b_act, s->b_up, M * F, st);
+                                         det ? 0 : (size_t)M * F, nullptr, 0);
+            multi3(L.gate, s->b_act, F, L.up, s->b_up, F, nullptr, nullptr, 0, det);
+            if (e == hipSuccess) e = launch_silu_mul(s->b_act, s->b_up, M * F, st);
         }
-        gemm(L.down, nullptr, s->b_act, F, s->b_hidden, H, OUT_ADD, down_split ? &s->xp : nullptr);
+        add_product(L.down, s->b_act, F, s->b_hidden, H);
     }
     if (!output) return e;  // a prompt chunk: K/V rows only
     // the final norm also clears the argmax keys; the output product stores
@@ -1301,7 +1381,7 @@ int ziggy_hip_session_verify(ZiggyHipSession *s, uint32_t current_token, const u
     for (uint32_t i = 0; i < M; i++)
         if (toks[i] >= s->embd.rows) return fail(err, err_len, ZIGGY_HIP_INVALID_ARGUMENT, "token id out of range");
     hipStream_t st = s->ctx->stream;
-    ZH_TRY(pass_alloc(s), "verify buffers");
+    ZH_TRY(pass_alloc(s, M), "verify buffers");
     ZH_TRY(hipMemcpyAsync(s->b_tokens, toks, M * 4, hipMemcpyHostToDevice, st), "verify tokens");
     ZH_TRY(pass_enqueue(s, s->b_tokens, (int)M, (int)s->position, true, st), "verify");
     unsigned long long keys[kVerifyMax];
