@@ -45,3 +45,28 @@ def test_prompt_rows_match_the_token_by_token_prompt(hip_ctx, ttype, rows):
         for a, b in zip(s.kv(1, pos), o.kv(1, pos)):
             assert rel_l2(a, b) < 1e-3
     s.close()
+
+
+# heads, kv heads, head size: query heads per kv head 8, 1, 3 (126 of a workgroup's 128 rows) and 4
+@pytest.mark.parametrize("heads,kv,hd", [(8, 1, 64), (4, 4, 128), (6, 2, 128), (8, 2, 96)])
+@pytest.mark.parametrize("second", [18, 90])
+def test_second_turn_attends_to_the_first(hip_ctx, heads, kv, hd, second):
+    """A short turn after a long one: its positions are split over workgroups whose partial results merge,
+    and its tiles start inside a page.  The bar is as above."""
+    print(f"second turn {heads}/{kv} heads of {hd}, {second} rows", flush=True)
+    spec = synth.small_spec(hidden=768, ffn=512, n_head=heads, n_kv=kv, head_dim=hd, default_type=Q8_0,
+                            attn_v_type=Q8_0, output_type=Q8_0, embd_type=Q8_0, context=700)
+    img = synth.build(spec, seed=23)
+    first, then = synth.prompt_tokens(1, 590, spec.vocab), synth.prompt_tokens(2, second, spec.vocab)
+    o = zo.Session(zo.Model(img.buf), context=spec.context, kv_f16=True)
+    for t in [*first, *then[:-1]]:
+        o.step_no_output(int(t))
+    want = o.step(int(then[-1]))
+    s = hip.Session(hip_ctx, img, context=spec.context)
+    s.generate(first, 0)
+    s.generate(then, 0)
+    assert rel_l2(s.logits(), want) < 1e-4
+    for pos in (590, 590 + second // 2, 590 + second - 2):
+        for a, b in zip(s.kv(1, pos), o.kv(1, pos)):
+            assert rel_l2(a, b) < 1e-3
+    s.close()

@@ -454,6 +454,11 @@ struct AttnParams {
 };
 constexpr uint32_t kPollEmpty = 0xFFFFFFFFu;  // a NaN pattern no arithmetic here produces
 hipError_t launch_attention(const AttnParams &p, hipStream_t s);
+// A prompt pass's attention (zh_pattn.hip): n_query queries in plain mode, each over the positions up
+// to its own (window_start 0), the K/V rows of all of them stored.  part: workspace (floats) for the
+// partial results where few queries leave CUs idle and the positions are split.
+bool prompt_attention_supported(int head_dim, int head_count, int head_count_kv);
+hipError_t launch_prompt_attention(const AttnParams &p, float *part, size_t part_floats, hipStream_t s);
 // A decode step's q/k/v projection (qkv: fused RMSNorm, up to three segments
 // in at most two formats, plain stores) and its single-query attention
 // (fused mode with the polled merge) in one launch (qkv_attn_kernel): the

@@ -901,8 +901,7 @@ static hipError_t pass_enqueue(ZiggyHipSession *s, const uint32_t *tokens, int M
 // Prompt rows per batched pass at most: a 4096-row product of a 4096-row matrix is 256 tiles of
 // 256 x 256, one per CU (Llama-8B-shaped 4096-token prompt, 4 layers: 46.6 ms in passes of 256).
 constexpr uint32_t kPrefillMax = 4096;
-// Passes of models with a matrix that the prompt products don't take (pgemm_supported), and the
-// attention launches of a pass, whose split partials are sized for this many queries.
+// Rows of the passes of models with a matrix that the prompt products don't take (pgemm_supported).
 constexpr uint32_t kPassBase = 256;
 // prompt rows per batched pass (ZIGGY_HIP_PREFILL_CHUNK, 16 .. 4096; a tuning knob)
 static uint32_t prefill_chunk() {
@@ -1065,7 +1064,7 @@ static hipError_t pass_alloc(ZiggyHipSession *s, uint32_t rows) {
         }
         if (attention_multi_supported((int)s->md.head_dim)) {
             const size_t slots = (size_t)s->md.head_count_kv *
-                                 attention_query_groups((int)s->md.head_count, (int)s->md.head_count_kv, (int)B);
+                                 attention_query_groups((int)s->md.head_count, (int)s->md.head_count_kv, (int)kVerifyMax);
             const size_t po = slots * s->max_splits * kMultiHeads * s->md.head_dim,
                          pml = slots * s->max_splits * kMultiHeads * 2;
             hipError_t e = hipMalloc((void **)&s->b_part_o, (po + pml) * 4);
@@ -1282,14 +1281,8 @@ static hipError_t pass_enqueue(ZiggyHipSession *s, const uint32_t *tokens, int M
             a.window_start = 0;
             a.scale = 1.0f / sqrtf((float)md.head_dim);
             a.max_splits = s->max_splits;
-            for (int m = 0; m < M && e == hipSuccess; m += (int)kPassBase) {
-                AttnParams c = a;
-                c.q = s->b_q + (size_t)m * Q;
-                c.out = s->b_attn + (size_t)m * Q;
-                c.position = pos + m;
-                c.n_query = std::min(M - m, (int)kPassBase);
-                e = launch_attention(c, st);
-            }
+            if (e == hipSuccess)
+                e = planes ? launch_prompt_attention(a, s->pg_part, kPgPart, st) : launch_attention(a, st);
         }
         // token by token where the multi-query kernel does not serve the shape (head_dim 256, the
         // vector kernel): never with the polled merge, which needs the matrix-core kernel too
