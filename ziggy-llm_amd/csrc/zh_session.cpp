@@ -1229,9 +1229,14 @@ static hipError_t pass_enqueue(ZiggyHipSession *s, const uint32_t *tokens, int M
     if (dn && e == hipSuccess) e = launch_zero_spans(clear_qkv, st);
     for (int l = 0; l < (int)md.block_count && e == hipSuccess; l++) {
         const LayerW &L = s->layers[l];
+        // A prompt chunk's rows leave nothing but their K/V rows: the last layer's queries and all
+        // that follows them have no reader (the prompt's last token runs through the step).
+        const bool kv_only = !output && l + 1 == (int)md.block_count && s->b_counters;
         if (dn) {
             const RowNorm rn{(const float *)L.attn_norm.p, ss_attn};
             multi3(L.q, s->b_q, Q, L.k, s->b_k, KV, &L.v, s->b_v, KV, false, s->b_hidden, &rn);
+        } else if (kv_only && norm_planes((const float *)L.attn_norm.p, {&L.k, &L.v})) {
+            multi3(L.k, s->b_k, KV, L.v, s->b_v, KV, nullptr, nullptr, 0, true);
         } else if (norm_planes((const float *)L.attn_norm.p, {&L.q, &L.k, &L.v})) {
             multi3(L.q, s->b_q, Q, L.k, s->b_k, KV, &L.v, s->b_v, KV, true);
         } else {
@@ -1272,6 +1277,7 @@ static hipError_t pass_enqueue(ZiggyHipSession *s, const uint32_t *tokens, int M
             a.out_stride = Q;
             e = dn ? launch_attention_prep(a, s->b_q, st, RowScale{ss_attn, H, eps}, clear_ffn)
                    : launch_attention_prep(a, s->b_q, st);
+            if (kv_only) break;
             // plain mode over the stored rows
             a.k_new = a.v_new = nullptr;
             a.out = s->b_attn;
