@@ -27,6 +27,9 @@ struct ZiggyHipContext {
     unsigned *counters = nullptr;
     // identity block table (kIdentityPages entries): the bridge-level attention's contiguous cache
     uint32_t *identity_pages = nullptr;
+    // pinned host words that small transfers pass through (kPinWords), read and written by kernels
+    // of this context's stream; free between calls, which synchronise
+    uint32_t *pin = nullptr;
     // RoPE denominators base^(2i / n_rot) per (base, n_rot) seen, computed on the host
     struct RopeTable {
         float base;
@@ -34,6 +37,9 @@ struct ZiggyHipContext {
         float *dev;
     } rope_tables[8] = {};
 };
+
+constexpr size_t kPinWords = 64u << 10;  // ZiggyHipContext::pin (256 KiB): kPinHead words for state
+constexpr size_t kPinHead = 1024;        // and flags, the rest for a call's values
 
 struct ZiggyHipBuffer {
     ZiggyHipContext *ctx = nullptr;
@@ -279,6 +285,14 @@ hipError_t launch_dequant(int fmt, const uint8_t *w, uint64_t stride, float *out
                           hipStream_t s);
 
 // small ops (zh_ops.hip)
+// Up to four spans of 32-bit words copied in one launch.  Between device and pinned host memory a
+// few KB take about 3 us this way; an asynchronous copy to or from pageable memory takes 8-15 us.
+struct CopySpans {
+    uint32_t *dst[4];
+    const uint32_t *src[4];
+    int n[4];
+};
+hipError_t launch_copy_spans(const CopySpans &c, hipStream_t s);
 hipError_t launch_rms_norm(const float *x, const float *w, float *out, int n, float eps, float off, hipStream_t s);
 hipError_t launch_rms_norm_per_head(const float *x, const float *w, float *out, int heads, int hd, float eps,
                                     float off, hipStream_t s);

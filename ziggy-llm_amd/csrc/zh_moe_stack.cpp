@@ -548,16 +548,35 @@ int ziggy_hip_moe_stack_forward(ZiggyHipMoeStack *s, const float *hidden_in, flo
     if (!s || !hidden_in || !hidden_out) return fail(err, err_len, ZIGGY_HIP_INVALID_ARGUMENT, "null argument");
     hipStream_t st = s->ctx->stream;
     const size_t H = s->d.hidden, K = s->d.expert_used_count, NL = s->layers.size();
-    ZH_TRY(hipMemcpyAsync(hidden_of(s, 0), hidden_in, H * 4, hipMemcpyHostToDevice, st), "MoE input");
-    ZH_TRY(hipGraphLaunch(s->graph, st), "MoE stack");
-    ZH_TRY(hipMemcpyAsync(hidden_out, s->hidden, H * 4, hipMemcpyDeviceToHost, st), "MoE output");
     std::vector<uint32_t> r;
-    if (selected || weights) {
-        r.resize(NL * s->route_stride);
-        ZH_TRY(hipMemcpyAsync(r.data(), s->route, r.size() * 4, hipMemcpyDeviceToHost, st), "MoE routing");
+    if (selected || weights) r.resize(NL * s->route_stride);
+    uint32_t *pin = s->ctx->pin, *values = pin + kPinHead;
+    if (H + r.size() <= kPinWords - kPinHead) {
+        // the rows, the routes and the error flag by way of the pinned words: one launch before the
+        // stack, one after it, one wait
+        memcpy(values, hidden_in, H * 4);
+        ZH_TRY(launch_copy_spans(CopySpans{{reinterpret_cast<uint32_t *>(hidden_of(s, 0))}, {values}, {(int)H}}, st),
+               "MoE input");
+        ZH_TRY(hipGraphLaunch(s->graph, st), "MoE stack");
+        const CopySpans out{{values, values + H, pin},
+                            {reinterpret_cast<const uint32_t *>(s->hidden), s->route,
+                             reinterpret_cast<const uint32_t *>(s->poll_err)},
+                            {(int)H, (int)r.size(), 1}};
+        ZH_TRY(launch_copy_spans(out, st), "MoE output");
+        ZH_TRY(hipStreamSynchronize(st), "MoE stack");
+        memcpy(hidden_out, values, H * 4);
+        if (!r.empty()) memcpy(r.data(), values + H, r.size() * 4);
+        if (pin[0])
+            if (int pe = poll_check_moe(s, err, err_len)) return pe;
+    } else {
+        ZH_TRY(hipMemcpyAsync(hidden_of(s, 0), hidden_in, H * 4, hipMemcpyHostToDevice, st), "MoE input");
+        ZH_TRY(hipGraphLaunch(s->graph, st), "MoE stack");
+        ZH_TRY(hipMemcpyAsync(hidden_out, s->hidden, H * 4, hipMemcpyDeviceToHost, st), "MoE output");
+        if (!r.empty())
+            ZH_TRY(hipMemcpyAsync(r.data(), s->route, r.size() * 4, hipMemcpyDeviceToHost, st), "MoE routing");
+        ZH_TRY(hipStreamSynchronize(st), "MoE stack");
+        if (int pe = poll_check_moe(s, err, err_len)) return pe;
     }
-    ZH_TRY(hipStreamSynchronize(st), "MoE stack");
-    if (int pe = poll_check_moe(s, err, err_len)) return pe;
     for (size_t l = 0; l < r.size() / s->route_stride; l++)
         for (size_t k = 0; k < K; k++) {
             const uint32_t *e = &r[l * s->route_stride + 2 * k];

@@ -108,6 +108,13 @@ __global__ void zero_spans_kernel(ZeroSpans z) {
         for (size_t i = gi; i < z.n[j]; i += nthr) z.p[j][i] = 0.f;
 }
 
+__global__ void copy_spans_kernel(CopySpans c) {
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+        for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < c.n[j]; i += gridDim.x * blockDim.x)
+            c.dst[j][i] = c.src[j][i];
+}
+
 __global__ void add_kernel(float *__restrict__ dst, const float *__restrict__ src, int n) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) dst[i] = dst[i] + src[i];
@@ -323,6 +330,17 @@ hipError_t launch_zero_spans(const ZeroSpans &z, hipStream_t s) {
 hipError_t launch_silu_mul(float *gate, const float *up, int n, hipStream_t s) {
     if (n <= 0) return hipSuccess;
     hipLaunchKernelGGL(silu_mul_kernel, dim3(cdiv(n, 256)), dim3(256), 0, s, gate, up, n);
+    return hipGetLastError();
+}
+hipError_t launch_copy_spans(const CopySpans &c, hipStream_t s) {
+    int most = 0;
+    for (int j = 0; j < 4; j++) {
+        if (c.n[j] < 0 || (c.n[j] && (!c.dst[j] || !c.src[j]))) return hipErrorInvalidValue;
+        most = c.n[j] > most ? c.n[j] : most;
+    }
+    if (!most) return hipSuccess;
+    const int blocks = cdiv(most, 256);
+    hipLaunchKernelGGL(copy_spans_kernel, dim3(blocks < 64 ? blocks : 64), dim3(256), 0, s, c);
     return hipGetLastError();
 }
 hipError_t launch_add(float *dst, const float *src, int n, hipStream_t s) {

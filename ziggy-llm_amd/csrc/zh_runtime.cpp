@@ -193,6 +193,7 @@ int ziggy_hip_create_context(int device_index, ZiggyHipContext **out_ctx, ZiggyH
     if (hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking) != hipSuccess ||
         hipEventCreate(&ctx->seq_begin) != hipSuccess || hipEventCreate(&ctx->seq_end) != hipSuccess ||
         hipMalloc(&ctx->scratch, kCtxScratch) != hipSuccess ||
+        hipHostMalloc((void **)&ctx->pin, kPinWords * 4, hipHostMallocCoherent) != hipSuccess ||
         hipMalloc((void **)&ctx->counters, kCtxCounters * sizeof(unsigned)) != hipSuccess ||
         hipMemset(ctx->counters, 0, kCtxCounters * sizeof(unsigned)) != hipSuccess ||
         hipMalloc((void **)&ctx->identity_pages, kIdentityPages * sizeof(uint32_t)) != hipSuccess ||
@@ -222,6 +223,7 @@ void ziggy_hip_destroy_context(ZiggyHipContext *ctx) {
     if (ctx->scratch) hipFree(ctx->scratch);
     if (ctx->counters) hipFree(ctx->counters);
     if (ctx->identity_pages) hipFree(ctx->identity_pages);
+    if (ctx->pin) hipHostFree(ctx->pin);
     if (ctx->seq_begin) hipEventDestroy(ctx->seq_begin);
     if (ctx->seq_end) hipEventDestroy(ctx->seq_end);
     if (ctx->stream) hipStreamDestroy(ctx->stream);

@@ -373,11 +373,33 @@ hipError_t launch_step(ZiggyHipSession *s, hipStream_t st) {
 
 // The polled attention's error flag: set when one of its waits ran out (the
 // step's outputs are then not valid); read after the stream is synchronized.
+constexpr size_t kPinFlag = 32, kPinState = 64;  // words of ZiggyHipContext::pin
 int poll_check(ZiggyHipSession *s, char *err, size_t err_len) {
     if (!s->attn_poll) return ZIGGY_HIP_OK;
     int flag = 0;
     ZH_TRY(hipMemcpy(&flag, s->poll_err, 4, hipMemcpyDeviceToHost), "poll flag");
     if (flag) return fail(err, err_len, ZIGGY_HIP_EXECUTION_FAILED, "an attention split never arrived (polled merge)");
+    return ZIGGY_HIP_OK;
+}
+// The host-driven step state to the device, by way of the pinned words.
+hipError_t upload_state(ZiggyHipSession *s, hipStream_t st) {
+    static_assert(sizeof(StepState) % 4 == 0 && sizeof(StepState) <= 4 * (kPinHead - kPinState), "fits the pinned words");
+    memcpy(s->ctx->pin + kPinState, s->st_host, sizeof(StepState));
+    return launch_copy_spans(CopySpans{{reinterpret_cast<uint32_t *>(s->st)}, {s->ctx->pin + kPinState}, {(int)(sizeof(StepState) / 4)}}, st);
+}
+// The step state, the error flag and n words of src (may be none) back, the stream synchronised:
+// st_host holds the state, the pinned words from kPinHead the values.
+int report(ZiggyHipSession *s, const void *src, int n, hipStream_t st, const char *what, char *err, size_t err_len) {
+    uint32_t *pin = s->ctx->pin;
+    pin[kPinFlag] = 0;
+    const CopySpans c{{pin + kPinState, pin + kPinFlag, pin + kPinHead},
+                      {reinterpret_cast<const uint32_t *>(s->st), reinterpret_cast<const uint32_t *>(s->poll_err),
+                       static_cast<const uint32_t *>(src)},
+                      {(int)(sizeof(StepState) / 4), s->attn_poll ? 1 : 0, n}};
+    ZH_TRY(launch_copy_spans(c, st), what);
+    ZH_TRY(hipStreamSynchronize(st), what);
+    memcpy(s->st_host, pin + kPinState, sizeof(StepState));
+    if (pin[kPinFlag]) return fail(err, err_len, ZIGGY_HIP_EXECUTION_FAILED, "an attention split never arrived (polled merge)");
     return ZIGGY_HIP_OK;
 }
 
@@ -667,9 +689,15 @@ int ziggy_hip_session_rewind(ZiggyHipSession *s, uint32_t position, char *err, s
 
 int ziggy_hip_session_begin_token(ZiggyHipSession *s, const float *hidden, char *err, size_t err_len) {
     if (!s || !hidden) return ZIGGY_HIP_INVALID_ARGUMENT;
-    ZH_TRY(hipMemcpyAsync(s->hidden, hidden, (size_t)s->md.embedding_length * 4, hipMemcpyHostToDevice,
-                          s->ctx->stream),
-           "begin_token");
+    const size_t n = s->md.embedding_length;
+    uint32_t *pin = s->ctx->pin + kPinHead;
+    if (n <= kPinWords - kPinHead) {
+        memcpy(pin, hidden, n * 4);
+        ZH_TRY(launch_copy_spans(CopySpans{{reinterpret_cast<uint32_t *>(s->hidden)}, {pin}, {(int)n}}, s->ctx->stream),
+               "begin_token");
+    } else {
+        ZH_TRY(hipMemcpyAsync(s->hidden, hidden, n * 4, hipMemcpyHostToDevice, s->ctx->stream), "begin_token");
+    }
     ZH_TRY(hipStreamSynchronize(s->ctx->stream), "begin_token");
     return ZIGGY_HIP_OK;
 }
@@ -713,9 +741,17 @@ int ziggy_hip_session_run_output_argmax(ZiggyHipSession *s, uint32_t *token, cha
 
 int ziggy_hip_session_read_hidden(ZiggyHipSession *s, float *out, char *err, size_t err_len) {
     if (!s || !out) return ZIGGY_HIP_INVALID_ARGUMENT;
-    ZH_TRY(hipMemcpyAsync(out, s->hidden, (size_t)s->md.embedding_length * 4, hipMemcpyDeviceToHost, s->ctx->stream),
-           "read_hidden");
+    const size_t n = s->md.embedding_length;
+    uint32_t *pin = s->ctx->pin + kPinHead;
+    const bool small = n <= kPinWords - kPinHead;
+    if (small)
+        ZH_TRY(launch_copy_spans(CopySpans{{pin}, {reinterpret_cast<const uint32_t *>(s->hidden)}, {(int)n}},
+                                 s->ctx->stream),
+               "read_hidden");
+    else
+        ZH_TRY(hipMemcpyAsync(out, s->hidden, n * 4, hipMemcpyDeviceToHost, s->ctx->stream), "read_hidden");
     ZH_TRY(hipStreamSynchronize(s->ctx->stream), "read_hidden");
+    if (small) memcpy(out, pin, n * 4);
     return ZIGGY_HIP_OK;
 }
 
@@ -727,17 +763,31 @@ int ziggy_hip_session_read_kv(ZiggyHipSession *s, uint32_t layer, uint32_t pos, 
                               size_t err_len) {
     if (!s || layer >= s->md.block_count || pos >= s->md.context_length || !k_out || !v_out)
         return ZIGGY_HIP_INVALID_ARGUMENT;
-    std::vector<__half> tmp(2 * (size_t)s->kv_size);
     const size_t base = kv_layer_base(s, (int)layer) + kv_row_host(s, pos) * s->kv_size;
-    ZH_TRY(hipMemcpyAsync(tmp.data(), s->kc + base, (size_t)s->kv_size * 2, hipMemcpyDeviceToHost, s->ctx->stream),
-           "read_kv");
-    ZH_TRY(hipMemcpyAsync(tmp.data() + s->kv_size, s->vc + base, (size_t)s->kv_size * 2, hipMemcpyDeviceToHost,
-                          s->ctx->stream),
-           "read_kv");
+    std::vector<__half> tmp;
+    const __half *rows = reinterpret_cast<const __half *>(s->ctx->pin + kPinHead);
+    if (s->kv_size % 2 == 0 && (size_t)s->kv_size <= kPinWords - kPinHead) {
+        const int words = s->kv_size / 2;
+        uint32_t *pin = s->ctx->pin + kPinHead;
+        ZH_TRY(launch_copy_spans(CopySpans{{pin, pin + words},
+                                           {reinterpret_cast<const uint32_t *>(s->kc + base),
+                                            reinterpret_cast<const uint32_t *>(s->vc + base)},
+                                           {words, words}},
+                                 s->ctx->stream),
+               "read_kv");
+    } else {
+        tmp.resize(2 * (size_t)s->kv_size);
+        rows = tmp.data();
+        ZH_TRY(hipMemcpyAsync(tmp.data(), s->kc + base, (size_t)s->kv_size * 2, hipMemcpyDeviceToHost, s->ctx->stream),
+               "read_kv");
+        ZH_TRY(hipMemcpyAsync(tmp.data() + s->kv_size, s->vc + base, (size_t)s->kv_size * 2, hipMemcpyDeviceToHost,
+                              s->ctx->stream),
+               "read_kv");
+    }
     ZH_TRY(hipStreamSynchronize(s->ctx->stream), "read_kv");
     for (int i = 0; i < s->kv_size; i++) {
-        k_out[i] = __half2float(tmp[i]);
-        v_out[i] = __half2float(tmp[s->kv_size + i]);
+        k_out[i] = __half2float(rows[i]);
+        v_out[i] = __half2float(rows[s->kv_size + i]);
     }
     return ZIGGY_HIP_OK;
 }
@@ -822,11 +872,9 @@ static int host_step(ZiggyHipSession *s, uint32_t token, bool output, uint32_t *
     h->out_flag = output ? 1 : 0;
     h->token = token;
     hipStream_t st = s->ctx->stream;
-    ZH_TRY(hipMemcpyAsync(s->st, h, sizeof(StepState), hipMemcpyHostToDevice, st), "step state");
+    ZH_TRY(upload_state(s, st), "step state");
     ZH_TRY(launch_step(s, st), "step graph");
-    if (output) ZH_TRY(hipMemcpyAsync(h, s->st, sizeof(StepState), hipMemcpyDeviceToHost, st), "step readback");
-    ZH_TRY(hipStreamSynchronize(st), "step");
-    if (int pe = poll_check(s, err, err_len)) return pe;
+    if (int re = report(s, nullptr, 0, st, "step", err, err_len)) return re;
     s->fed.resize(s->position);
     s->fed.push_back(token);
     s->position++;
@@ -887,8 +935,10 @@ int ziggy_hip_session_step_shortlist(ZiggyHipSession *s, uint32_t token, uint32_
     hipStream_t sm = s->ctx->stream;
     ZH_TRY(enqueue_output_logits(s, sm), "shortlist output");
     ZH_TRY(launch_shortlist(s->logits, V, (int)count, s->sl_keys, s->sl_entries, sm), "shortlist");
-    ZH_TRY(hipMemcpyAsync(out, s->sl_entries, (size_t)count * 8, hipMemcpyDeviceToHost, sm), "shortlist readback");
+    uint32_t *pin = s->ctx->pin + kPinHead;
+    ZH_TRY(launch_copy_spans(CopySpans{{pin}, {s->sl_entries}, {(int)(2 * count)}}, sm), "shortlist readback");
     ZH_TRY(hipStreamSynchronize(sm), "shortlist");
+    memcpy(out, pin, (size_t)count * 8);
     s->logits_valid = true;
     return ZIGGY_HIP_OK;
 }
@@ -978,7 +1028,12 @@ int ziggy_hip_session_generate(ZiggyHipSession *s, const uint32_t *prompt, uint3
         int bst = build_graph(s, err, err_len);
         if (bst) return bst;
     }
-    ZH_TRY(hipMemcpyAsync(s->prompt, prompt, (size_t)prompt_len * 4, hipMemcpyHostToDevice, st), "prompt upload");
+    if (prompt_len <= kPinWords - kPinHead) {
+        memcpy(s->ctx->pin + kPinHead, prompt, (size_t)prompt_len * 4);
+        ZH_TRY(launch_copy_spans(CopySpans{{s->prompt}, {s->ctx->pin + kPinHead}, {(int)prompt_len}}, st), "prompt upload");
+    } else {
+        ZH_TRY(hipMemcpyAsync(s->prompt, prompt, (size_t)prompt_len * 4, hipMemcpyHostToDevice, st), "prompt upload");
+    }
     // every prompt row but the last in batched passes of up to prefill_chunk()
     // tokens (GEMMs on the matrix cores, multi-query causal attention), the
     // last one through the step graph for its logits; the reference feeds
@@ -993,7 +1048,7 @@ int ziggy_hip_session_generate(ZiggyHipSession *s, const uint32_t *prompt, uint3
     h->step = (int)n_batched;  // the graph's first step takes prompt[n_batched]
     h->n_prompt = (int)prompt_len;
     h->n_gen = (int)steps;
-    ZH_TRY(hipMemcpyAsync(s->st, h, sizeof(StepState), hipMemcpyHostToDevice, st), "step state");
+    ZH_TRY(upload_state(s, st), "step state");
     ZH_TRY(hipStreamSynchronize(st), "generate setup");
     const uint64_t tp0 = now_ns();
     const uint32_t chunk = std::min(prefill_chunk(), s->pass_rows);
@@ -1009,12 +1064,13 @@ int ziggy_hip_session_generate(ZiggyHipSession *s, const uint32_t *prompt, uint3
     const uint64_t t0 = now_ns();
     for (uint32_t i = 0; i < steps; i++) ZH_TRY(launch_step(s, st), "decode step");
     ZH_TRY(hipEventRecord(s->ctx->seq_end, st), "generate");
-    ZH_TRY(hipStreamSynchronize(st), "decode");
+    const bool small = steps <= kPinWords - kPinHead;
+    const int re = report(s, s->history, small ? (int)steps : 0, st, "decode", err, err_len);
     const uint64_t t1 = now_ns();
-    if (steps) ZH_TRY(hipMemcpy(out_tokens, s->history, (size_t)steps * 4, hipMemcpyDeviceToHost), "history");
-    ZH_TRY(hipMemcpy(h, s->st, sizeof(StepState), hipMemcpyDeviceToHost), "state readback");
+    if (re) return re;
+    if (steps && small) memcpy(out_tokens, s->ctx->pin + kPinHead, (size_t)steps * 4);
+    if (!small) ZH_TRY(hipMemcpy(out_tokens, s->history, (size_t)steps * 4, hipMemcpyDeviceToHost), "history");
     if (h->error) return fail(err, err_len, ZIGGY_HIP_EXECUTION_FAILED, "a generated token was out of range");
-    if (int pe = poll_check(s, err, err_len)) return pe;
     // rows of the prompt, then of each generated token but the last (still pending)
     s->fed.resize(s->position);
     s->fed.insert(s->fed.end(), prompt, prompt + prompt_len);
@@ -1381,11 +1437,16 @@ int ziggy_hip_session_verify(ZiggyHipSession *s, uint32_t current_token, const u
         if (toks[i] >= s->embd.rows) return fail(err, err_len, ZIGGY_HIP_INVALID_ARGUMENT, "token id out of range");
     hipStream_t st = s->ctx->stream;
     ZH_TRY(pass_alloc(s, M), "verify buffers");
-    ZH_TRY(hipMemcpyAsync(s->b_tokens, toks, M * 4, hipMemcpyHostToDevice, st), "verify tokens");
+    uint32_t *pin = s->ctx->pin + kPinHead;
+    memcpy(pin, toks, M * 4);
+    ZH_TRY(launch_copy_spans(CopySpans{{s->b_tokens}, {pin}, {(int)M}}, st), "verify tokens");
     ZH_TRY(pass_enqueue(s, s->b_tokens, (int)M, (int)s->position, true, st), "verify");
     unsigned long long keys[kVerifyMax];
-    ZH_TRY(hipMemcpyAsync(keys, s->b_argmax, M * 8, hipMemcpyDeviceToHost, st), "verify readback");
+    ZH_TRY(launch_copy_spans(CopySpans{{pin + 2 * kVerifyMax}, {reinterpret_cast<const uint32_t *>(s->b_argmax)}, {(int)(2 * M)}},
+                             st),
+           "verify readback");
     ZH_TRY(hipStreamSynchronize(st), "verify");
+    memcpy(keys, pin + 2 * kVerifyMax, M * 8);
     // verifyDraftTokensSequential (model/loader.zig:1131-1151): emit predictions until one
     // differs from its draft; all drafts accepted adds the bonus prediction
     for (uint32_t i = 0; i < M; i++) out_predicted[i] = 0xFFFFFFFFu - (uint32_t)(keys[i] & 0xFFFFFFFFull);
