@@ -70,3 +70,28 @@ def test_second_turn_attends_to_the_first(hip_ctx, heads, kv, hd, second):
         for a, b in zip(s.kv(1, pos), o.kv(1, pos)):
             assert rel_l2(a, b) < 1e-3
     s.close()
+
+
+@pytest.mark.parametrize("ttype", [Q4_K, Q6_K, Q8_0, IQ4_XS, Q3_K], ids=lambda t: TYPE_NAMES[t])
+def test_largest_tiles_match_the_step_path(hip_ctx, ttype):
+    """4096-row matrices and 3841 prompt rows: tiles of 256 x 256, the last of them one row.  Against the same
+    prompt token by token through the decode step, which has the oracle's bars of 1e-4 and 1e-3: twice those."""
+    print(f"largest tiles {TYPE_NAMES[ttype]}", flush=True)
+    spec = synth.small_spec(hidden=4096, ffn=512, n_head=32, n_kv=32, head_dim=128, default_type=ttype,
+                            attn_v_type=ttype, output_type=Q8_0, embd_type=Q8_0, context=3904)
+    img = synth.build(spec, seed=29)
+    prompt = synth.prompt_tokens(3, 3842, spec.vocab)
+    s = hip.Session(hip_ctx, img, context=spec.context)
+    s.generate(prompt, 0)
+    got = s.logits()
+    at = (0, 255, 256, 2000, 3839, 3840)
+    rows = [s.kv(1, p) for p in at]
+    s.rewind(0)
+    for t in prompt[:-1]:
+        s.step_no_output(int(t))
+    s.step_greedy(int(prompt[-1]))
+    assert rel_l2(got, s.logits()) < 2e-4
+    for p, kv in zip(at, rows):
+        for a, b in zip(kv, s.kv(1, p)):
+            assert rel_l2(a, b) < 2e-3
+    s.close()
