@@ -30,6 +30,10 @@ struct ZiggyHipContext {
     // pinned host words that small transfers pass through (kPinWords), read and written by kernels
     // of this context's stream; free between calls, which synchronise
     uint32_t *pin = nullptr;
+    // a second stream for work that runs beside the first within one call: it waits for side_fork
+    // (recorded on `stream`), and `stream` waits for side_join before the call ends
+    hipStream_t side = nullptr;
+    hipEvent_t side_fork = nullptr, side_join = nullptr;
     // RoPE denominators base^(2i / n_rot) per (base, n_rot) seen, computed on the host
     struct RopeTable {
         float base;

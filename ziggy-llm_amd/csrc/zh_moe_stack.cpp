@@ -79,6 +79,7 @@ void free_stack(ZiggyHipMoeStack *s) {
     if (s->ctx) {
         hipSetDevice(s->ctx->device);
         hipStreamSynchronize(s->ctx->stream);
+        hipStreamSynchronize(s->ctx->side);
     }
     if (s->graph) hipGraphExecDestroy(s->graph);
     for (void *p : s->allocs) hipFree(p);
@@ -294,8 +295,21 @@ hipError_t enqueue_prefill_layer(ZiggyHipMoeStack *s, int l, int M, hipStream_t 
         float *ys[1] = {y};
         const int Ns[1] = {n};
         return launch_pgemm((int)w.type, 1, ws, w2 ? w2->p : nullptr, ys, Ns, Ns, w.stride, s->p_hp, M, (int)w.cols, out,
-                            s->p_part, kSharedPart, st);
+                            s->p_part, kSharedPart, s->ctx->side);
     };
+    // The shared expert's launches (about 60 us at 512 rows, too few workgroups to fill the chip) run
+    // beside the router, the routing and the routed experts, which neither read nor write its buffers;
+    // the combine waits for them, and so does the next layer's norm, which writes the planes again.
+    // (512 rows, 4 layers of the 256-expert stack, the whole call: 2003 -> 1844 us)
+    bool forked = false;
+    if (e == hipSuccess && sh_planes) {
+        e = hipEventRecord(s->ctx->side_fork, st);
+        if (e == hipSuccess) e = hipStreamWaitEvent(s->ctx->side, s->ctx->side_fork, 0);
+        forked = e == hipSuccess;
+        if (e == hipSuccess) e = sh_product(L.gate_sh, &L.up_sh, s->p_act_sh, SF, OUT_SWIGLU);
+        if (e == hipSuccess) e = launch_row_planes(s->p_act_sh, SF, M, SF, s->p_hp, s->ctx->side);
+        if (e == hipSuccess) e = sh_product(L.down_sh, nullptr, s->p_sh, H, OUT_STORE);
+    }
     // the shared gate row, stored right after the router's rows, is row E of one launch
     const bool gate_row_next = s->shared_gate && L.gate_inp_sh.p == L.router.p + (uint64_t)E * L.router.stride &&
                                L.gate_inp_sh.stride == L.router.stride;
@@ -315,11 +329,7 @@ hipError_t enqueue_prefill_layer(ZiggyHipMoeStack *s, int l, int M, hipStream_t 
         e = launch_gemm_grouped(L.gate.type, L.gate.p, L.up.p, L.gate.stride, (uint64_t)FF * L.gate.stride,
                                 s->p_normed, H, K, s->p_act, FF, FF, H, OUT_SWIGLU, s->p_tiles, s->p_list,
                                 s->p_ntiles, max_tiles, st);
-    if (e == hipSuccess && sh_planes) {
-        e = sh_product(L.gate_sh, &L.up_sh, s->p_act_sh, SF, OUT_SWIGLU);
-        if (e == hipSuccess) e = launch_row_planes(s->p_act_sh, SF, M, SF, s->p_hp, st);
-        if (e == hipSuccess) e = sh_product(L.down_sh, nullptr, s->p_sh, H, OUT_STORE);
-    } else if (e == hipSuccess && s->shared) {
+    if (e == hipSuccess && s->shared && !sh_planes) {
         e = launch_gemm(L.gate_sh.type, L.gate_sh.p, L.up_sh.p, L.gate_sh.stride, s->p_normed, H, s->p_act_sh, SF, M,
                         SF, H, OUT_SWIGLU, nullptr, st);
     }
@@ -330,6 +340,11 @@ hipError_t enqueue_prefill_layer(ZiggyHipMoeStack *s, int l, int M, hipStream_t 
     if (e == hipSuccess && s->shared && !sh_planes)
         e = launch_gemm(L.down_sh.type, L.down_sh.p, nullptr, L.down_sh.stride, s->p_act_sh, SF, s->p_sh, H, M, H, SF,
                         OUT_STORE, nullptr, st);
+    if (forked) {  // also after a failed launch: nothing on the stream outlives the side's work
+        hipError_t j = hipEventRecord(s->ctx->side_join, s->ctx->side);
+        if (j == hipSuccess) j = hipStreamWaitEvent(st, s->ctx->side_join, 0);
+        if (e == hipSuccess) e = j;
+    }
     if (e == hipSuccess)
         e = launch_moe_combine(s->p_hidden, s->p_tmp, route, H, K, s->shared ? 1 : 0, st, M,
                                s->shared ? s->p_sh : nullptr);

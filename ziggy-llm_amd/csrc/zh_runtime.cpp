@@ -191,6 +191,9 @@ int ziggy_hip_create_context(int device_index, ZiggyHipContext **out_ctx, ZiggyH
     ctx->info.clock_khz = (uint32_t)prop.clockRate;
     ctx->info.l2_bytes = (uint32_t)prop.l2CacheSize;
     if (hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking) != hipSuccess ||
+        hipStreamCreateWithFlags(&ctx->side, hipStreamNonBlocking) != hipSuccess ||
+        hipEventCreateWithFlags(&ctx->side_fork, hipEventDisableTiming) != hipSuccess ||
+        hipEventCreateWithFlags(&ctx->side_join, hipEventDisableTiming) != hipSuccess ||
         hipEventCreate(&ctx->seq_begin) != hipSuccess || hipEventCreate(&ctx->seq_end) != hipSuccess ||
         hipMalloc(&ctx->scratch, kCtxScratch) != hipSuccess ||
         hipHostMalloc((void **)&ctx->pin, kPinWords * 4, hipHostMallocCoherent) != hipSuccess ||
@@ -218,6 +221,7 @@ void ziggy_hip_destroy_context(ZiggyHipContext *ctx) {
     if (!ctx) return;
     hipSetDevice(ctx->device);
     if (ctx->stream) hipStreamSynchronize(ctx->stream);
+    if (ctx->side) hipStreamSynchronize(ctx->side);
     for (auto &t : ctx->rope_tables)
         if (t.dev) hipFree(t.dev);
     if (ctx->scratch) hipFree(ctx->scratch);
@@ -226,6 +230,9 @@ void ziggy_hip_destroy_context(ZiggyHipContext *ctx) {
     if (ctx->pin) hipHostFree(ctx->pin);
     if (ctx->seq_begin) hipEventDestroy(ctx->seq_begin);
     if (ctx->seq_end) hipEventDestroy(ctx->seq_end);
+    if (ctx->side_fork) hipEventDestroy(ctx->side_fork);
+    if (ctx->side_join) hipEventDestroy(ctx->side_join);
+    if (ctx->side) hipStreamDestroy(ctx->side);
     if (ctx->stream) hipStreamDestroy(ctx->stream);
     delete ctx;
 }
