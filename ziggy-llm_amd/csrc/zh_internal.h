@@ -363,7 +363,7 @@ hipError_t launch_norm_planes(const float *x, const float *w, float *out, int ro
 bool pgemm_supported(int fmt, int K, const void *w, uint64_t stride);
 hipError_t launch_pgemm(int fmt, int nseg, const uint8_t *const *w, const uint8_t *w2, float *const *y, const int *ldy,
                         const int *N, uint64_t stride, const HPlanes &xp, int M, int K, int out, float *part,
-                        size_t part_floats, hipStream_t s, int force_cfg = -1, int force_ks = 0);
+                        size_t part_floats, hipStream_t s);
 // MFMA GEMM for M >= 8 tokens (zh_gemm.hip): Y[m][n] (=, +=) sum_k W[n][k] X[m][k]
 // (OUT_STORE / OUT_ADD / OUT_SWIGLU with w2 / OUT_ARGMAX into argmax[M]).
 // max_split bounds the reduction split of the exact-code kernel, whose

@@ -555,7 +555,7 @@ bool pgemm_supported(int fmt, int K, const void *w, uint64_t stride) {
 
 hipError_t launch_pgemm(int fmt, int nseg, const uint8_t *const *w, const uint8_t *w2, float *const *y, const int *ldy,
                         const int *N, uint64_t stride, const HPlanes &xp, int M, int K, int out, float *part,
-                        size_t part_floats, hipStream_t s, int force_cfg, int force_ks) {
+                        size_t part_floats, hipStream_t s) {
     if (nseg < 1 || nseg > 3 || M < 1 || !xp.x || !xp.xs || !xp.scale || (out == OUT_SWIGLU && (nseg != 1 || !w2)) ||
         (out != OUT_STORE && out != OUT_ADD && out != OUT_SWIGLU))
         return hipErrorInvalidValue;
@@ -576,14 +576,12 @@ hipError_t launch_pgemm(int fmt, int nseg, const uint8_t *const *w, const uint8_
     int cfg = 0, ks = 1;
     double best = 0.0;
     for (int c = 0; c < 3; c++) {
-        if (force_cfg >= 0 && c != force_cfg) continue;
         const PTile &t = kPTiles[c];
         const int tno = t.tn / mats;
         long long tiles = 0;
         for (int i = 0; i < nseg; i++) tiles += (N[i] + tno - 1) / tno;
         tiles *= (M + t.tm - 1) / t.tm;
         for (int k = 1; k <= 16 && k <= K / 256; k *= 2) {
-            if (force_ks > 0 && k != force_ks) continue;
             if (k > 1 && (!part || p.msum * k > part_floats)) break;
             static const double one[] = {1.68, 0.85, 0.6}, full[] = {2.43, 1.49, 0.8};
             const long long wgs = tiles * k, slots = 256 * t.per_cu, rounds = (wgs + slots - 1) / slots;
