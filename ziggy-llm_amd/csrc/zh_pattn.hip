@@ -10,13 +10,17 @@
 // holds 16 positions of one row, so maximum, weights and sum stay in the lane (one exchange with
 // the lane 32 on per tile), and O[dim][row] = V^T P^T takes the weights as they lie, in two pieces.
 // The order of a product's reduction index is free as long as both operands share it: the weights'
-// own.  Weights and sums are binary32, the pieces 2^-21 of a weight.
+// own.  Weights and sums are binary32.  The pieces are of the weights times 2^14 (outputs and sums
+// carry the factor, which their quotient drops): both rounded to nearest, they hold a weight to 2^-22
+// of itself, or to 2^-39 of the row's largest, so that thousands of small weights beside one large
+// keep their sum.
 //
 // What bounds it: per tile and wavefront 64 matrix products (2048 cycles) and about 300 vector
 // instructions (1200), two wavefronts per SIMD; 16384 queries x 32 heads over 16384 positions (head
-// size 128) take 4.1 ms a layer, 1080 TFLOP/s of issued matrix work (the library's f16 product
-// reaches 1180-1230 on the same card); the kernel before it, whose workgroups took four queries
-// each and read the range again for every four, 15 ms.
+// size 128) take 4.1 ms a layer (4.3 on another card), 1080 TFLOP/s of issued matrix work (the
+// library's f16 product reaches 1180-1230 on the same card); the kernel before it, whose workgroups
+// took four queries each and read the range again for every four, 15 ms.  Scaling the weights' pieces
+// as it does costs 0.7% (1074 -> 1081 us over four passes of a layer), scaling the weights 5%.
 //
 // Few queries over many positions leave CUs idle: their positions are split over up to 16
 // workgroups and a second launch merges.  (20 / 64 / 256 / 600 queries after 4000 positions, one
@@ -34,6 +38,7 @@ typedef _Float16 ph8 __attribute__((ext_vector_type(8)));
 typedef float pf16 __attribute__((ext_vector_type(16)));
 
 constexpr int kPaRows = 128;  // query x head rows of a workgroup, 32 per wavefront
+constexpr float kPaWeight = 16384.f;  // of the largest weight: its pieces below binary16's 65504
 
 struct PAttnParams {
     const float *q;
@@ -202,8 +207,9 @@ template <int HD> __global__ void __launch_bounds__(256, 2) pattn_kernel(PAttnPa
             for (int i = 0; i < 8; i++) {
                 const float a = __builtin_amdgcn_exp2f(s[pt][2 * i] - mf), b = __builtin_amdgcn_exp2f(s[pt][2 * i + 1] - mf);
                 l += a + b;
-                const auto h = __builtin_amdgcn_cvt_pkrtz(a, b);
-                const auto w = __builtin_amdgcn_cvt_pkrtz(a - (float)h[0], b - (float)h[1]);
+                // (the packed multiply is exact, and half the instructions of scaling a and b)
+                const ph2 h = ph2{(_Float16)a, (_Float16)b} * (_Float16)kPaWeight;
+                const ph2 w = {(_Float16)fmaf(a, kPaWeight, -(float)h[0]), (_Float16)fmaf(b, kPaWeight, -(float)h[1])};
                 hi[i] = __builtin_bit_cast(uint32_t, h);
                 lo[i] = __builtin_bit_cast(uint32_t, w);
             }
@@ -249,7 +255,7 @@ template <int HD> __global__ void __launch_bounds__(256, 2) pattn_kernel(PAttnPa
         tile(c0, t);
         if (t + 1 < nt) tile(c1, t + 1);
     }
-    l = pair_sum(l);
+    l = pair_sum(l) * kPaWeight;  // as the outputs
     if (!valid) return;
     const bool split = ks > 1;
     const float inv = split ? 1.f : 1.f / l;
