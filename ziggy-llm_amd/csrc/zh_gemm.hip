@@ -214,8 +214,9 @@ template <int F> static GemmKernel pick_grouped(int out) {
 }
 
 // ZIGGY_HIP_QGEMM=0 keeps every M >= 8 product on this file's kernel (the
-// exact-code kernel of zh_qgemm.hip otherwise takes the quantized formats).
-static bool qgemm_enabled() {
+// exact-code kernels of zh_qgemm.hip and zh_pgemm.hip otherwise take the
+// quantized formats).
+bool qgemm_enabled() {
     static const bool on = [] {
         const char *e = getenv("ZIGGY_HIP_QGEMM");
         return !(e && e[0] == '0');

@@ -398,6 +398,7 @@ hipError_t launch_gemm_grouped(int fmt, const uint8_t *w, const uint8_t *w2, uin
                                const float *x, int ldx, int x_div, float *y, int ldy, int N, int K, int out,
                                const int *tiles, const int *list, const int *ntiles, int max_tiles, hipStream_t s);
 // Exact-code MFMA kernel (zh_qgemm.hip) for the quantized formats, K a multiple of 256.
+bool qgemm_enabled();  // unless ZIGGY_HIP_QGEMM=0
 bool qgemm_supported(int fmt, int K, const void *w, const void *w2, uint64_t stride, uint64_t expert_stride);
 hipError_t launch_qgemm(int fmt, const uint8_t *w, const uint8_t *w2, uint64_t stride, const float *x, int ldx,
                         float *y, int ldy, int M, int N, int K, int out, unsigned long long *argmax, hipStream_t s,

@@ -550,7 +550,7 @@ template <int OUT> static PGemmKernel pick_pgf(int fmt, int cfg) {
 }
 
 bool pgemm_supported(int fmt, int K, const void *w, uint64_t stride) {
-    return qgemm_supported(fmt, K, w, nullptr, stride, 0);
+    return qgemm_enabled() && qgemm_supported(fmt, K, w, nullptr, stride, 0);
 }
 
 hipError_t launch_pgemm(int fmt, int nseg, const uint8_t *const *w, const uint8_t *w2, float *const *y, const int *ldy,

@@ -1173,7 +1173,8 @@ static hipError_t pass_alloc(ZiggyHipSession *s, uint32_t rows) {
 // K/V row in order), o_proj / gate-up / down GEMMs with the residual adds,
 // final norm and the output GEMM fused with a per-token argmax.
 // ZIGGY_HIP_VERIFY_SWIGLU=fused keeps gate/up as one SWIGLU product (its
-// reduction never splits); by default they are two products and SiLU * up.
+// reduction never splits); by default they are two products and SiLU * up,
+// but for the products from planes, which are one in any case.
 static bool verify_fused_swiglu() {
     static const bool f = [] {
         const char *e = getenv("ZIGGY_HIP_VERIFY_SWIGLU");
@@ -1387,10 +1388,6 @@ static hipError_t pass_enqueue(ZiggyHipSession *s, const uint32_t *tokens, int M
             const RowNorm rn{(const float *)L.ffn_norm.p, ss_ffn};
             multi3(L.gate, s->b_act, F, L.up, s->b_up, F, nullptr, nullptr, 0, false, s->b_hidden, &rn);
             if (e == hipSuccess) e = launch_silu_mul_rows(s->b_act, s->b_up, M, F, RowScale{ss_ffn, H, eps}, clear_qkv, st);
-        } else if (fused_swiglu && !planes && L.gate.type == L.up.type) {
-            if (e == hipSuccess)
-                e = launch_rms_norm_rows(s->b_hidden, (const float *)L.ffn_norm.p, s->b_normed, M, H, eps, st);
-            gemm(L.gate, &L.up, s->b_normed, H, s->b_act, F, OUT_SWIGLU);
         } else if (planes && pg_ok(L.gate) && pg_ok(L.up) && L.gate.type == L.up.type && L.gate.stride == L.up.stride) {
             // both products of a row and SiLU(gate) * up in one launch
             norm_planes((const float *)L.ffn_norm.p, {&L.gate, &L.up});
@@ -1398,6 +1395,10 @@ static hipError_t pass_enqueue(ZiggyHipSession *s, const uint32_t *tokens, int M
             float *ys[1] = {s->b_act};
             const int lds[1] = {F};
             pgemm(1, d, &L.up, ys, lds, OUT_SWIGLU);
+        } else if (fused_swiglu && L.gate.type == L.up.type) {
+            if (e == hipSuccess)
+                e = launch_rms_norm_rows(s->b_hidden, (const float *)L.ffn_norm.p, s->b_normed, M, H, eps, st);
+            gemm(L.gate, &L.up, s->b_normed, H, s->b_act, F, OUT_SWIGLU);
         } else {
             // gate and up (prompt chunks: stores; verify passes: onto rows
             // the norm clears, each product may split its reduction), then
