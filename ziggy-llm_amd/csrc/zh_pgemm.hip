@@ -437,10 +437,13 @@ __global__ void __launch_bounds__(64 * NM * NN, 2) pgemm_kernel(PGemmParams p) {
         __builtin_amdgcn_sched_barrier(0);
         if (!first && more) {
             store(o, s + 1);
+            // the copies have landed before the next codes are asked for, which may then stay on their
+            // way over the barrier
+            __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+            __builtin_amdgcn_sched_barrier(0);
             load_b(min(s + 2, S - 1));
             __builtin_amdgcn_sched_barrier(0);
-            // all but the two newest loads: load_b issues at least two after load_a's
-            __builtin_amdgcn_s_waitcnt(0x72);
+            __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
         } else {
             __builtin_amdgcn_s_waitcnt(0x70);
         }
