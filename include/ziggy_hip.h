@@ -374,6 +374,18 @@ typedef struct {
 int ziggy_hip_probe_row_load(ZiggyHipContext *ctx, uint32_t reps, ZiggyHipRowLoadProbe *out, char *error_message,
                              size_t error_message_len);
 
+typedef struct {
+    uint32_t tokens, rows;  /* tile of a workgroup (of gate and up rows together, for a pair) */
+    uint32_t split;         /* workgroups that share a tile's reduction */
+} ZiggyHipPromptTiles;
+/* The tile and the reduction split that a prompt pass's product of `tokens`
+ * token rows takes: up to three matrices of rows[i] x cols (or, with pair, gate
+ * and up of rows[0] each).  Host arithmetic, no device.  workspace_floats: of
+ * the split's partial results (a session's passes: 16 << 20). */
+int ziggy_hip_probe_prompt_tiles(const uint32_t *rows, uint32_t count, uint32_t tokens, uint32_t cols, int pair,
+                                 size_t workspace_floats, ZiggyHipPromptTiles *out, char *error_message,
+                                 size_t error_message_len);
+
 /* Kernels of one decode step, for ziggy_hip_session_time_kernel. */
 enum {
     ZIGGY_HIP_KERNEL_QKV = 0,      /* fused RMSNorm + q/k/v projections */

@@ -74,7 +74,8 @@ def test_second_turn_attends_to_the_first(hip_ctx, heads, kv, hd, second):
 
 @pytest.mark.parametrize("ttype", [Q4_K, Q6_K, Q8_0, IQ4_XS, Q3_K], ids=lambda t: TYPE_NAMES[t])
 def test_largest_tiles_match_the_step_path(hip_ctx, ttype):
-    """4096-row matrices and 3841 prompt rows: tiles of 256 x 256, the last of them one row.  Against the same
+    """4096-row matrices and 3841 prompt rows: tiles of 256 x 256, the last of them one row (gate and up, of 512
+    rows, take smaller ones; test_tiles_and_splits_match_the_step_path has theirs).  Against the same
     prompt token by token through the decode step, which has the oracle's bars of 1e-4 and 1e-3: twice those."""
     print(f"largest tiles {TYPE_NAMES[ttype]}", flush=True)
     spec = synth.small_spec(hidden=4096, ffn=512, n_head=32, n_kv=32, head_dim=128, default_type=ttype,
@@ -93,5 +94,42 @@ def test_largest_tiles_match_the_step_path(hip_ctx, ttype):
     assert rel_l2(got, s.logits()) < 2e-4
     for p, kv in zip(at, rows):
         for a, b in zip(kv, s.kv(1, p)):
+            assert rel_l2(a, b) < 2e-3
+    s.close()
+
+
+# hidden, feed-forward, rows in the pass and the tile and split that the named product takes there
+PLANS = [(4096, 2048, 3841, {"gate_up": (256, 256, 1)}), (4096, 1024, 3841, {"gate_up": (256, 256, 2)}),
+         (4096, 2048, 257, {"gate_up": (256, 256, 8), "o": (256, 256, 8)}), (4096, 2048, 33, {"gate_up": (64, 128, 16)}),
+         (2048, 5632, 513, {"gate_up": (128, 128, 1), "down": (256, 256, 8)}), (2048, 2048, 2049, {"qkv": (128, 128, 1)})]
+
+
+@pytest.mark.parametrize("ttype", [Q4_K, Q6_K, Q8_0, IQ4_XS, Q3_K], ids=lambda t: TYPE_NAMES[t])
+@pytest.mark.parametrize("hidden,ffn,rows,plan", PLANS, ids=lambda v: str(v) if isinstance(v, int) else "")
+def test_tiles_and_splits_match_the_step_path(hip_ctx, ttype, hidden, ffn, rows, plan):
+    """Each tile size with gate and up paired, with and without a split.  The plan is asserted, so that a change
+    of the estimate's constants can't drop one unseen.  The bars are as above."""
+    print(f"tiles {TYPE_NAMES[ttype]} {hidden}/{ffn} rows {rows}", flush=True)
+    heads = hidden // 128
+    takes = {"qkv": hip.prompt_tiles([hidden, hidden // 4, hidden // 4], rows, hidden),
+             "o": hip.prompt_tiles([hidden], rows, hidden), "gate_up": hip.prompt_tiles([ffn], rows, hidden, True),
+             "down": hip.prompt_tiles([hidden], rows, ffn)}
+    assert {k: takes[k] for k in plan} == plan
+    spec = synth.small_spec(hidden=hidden, ffn=ffn, n_head=heads, n_kv=heads // 4, head_dim=128, default_type=ttype,
+                            attn_v_type=ttype, output_type=Q8_0, embd_type=Q8_0, context=rows + 63)
+    img = synth.build(spec, seed=31)
+    prompt = synth.prompt_tokens(4, rows + 1, spec.vocab)
+    s = hip.Session(hip_ctx, img, context=spec.context)
+    s.generate(prompt, 0)
+    got = s.logits()
+    at = (0, rows // 2, rows - 2, rows - 1)
+    kv = [s.kv(1, p) for p in at]
+    s.rewind(0)
+    for t in prompt[:-1]:
+        s.step_no_output(int(t))
+    s.step_greedy(int(prompt[-1]))
+    assert rel_l2(got, s.logits()) < 2e-4
+    for p, row in zip(at, kv):
+        for a, b in zip(row, s.kv(1, p)):
             assert rel_l2(a, b) < 2e-3
     s.close()

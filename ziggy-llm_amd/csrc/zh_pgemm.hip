@@ -563,6 +563,33 @@ template <int OUT> static PGemmKernel pick_pgf(int fmt, int cfg) {
     }
 }
 
+struct PgPlan {
+    int cfg, ks;  // tile (kPTiles), reduction split
+};
+static PgPlan pgemm_plan(int nseg, const int *N, int M, int K, int mats, size_t part_floats) {
+    size_t msum = 0;  // partial results of one split
+    for (int i = 0; i < nseg; i++) msum += (size_t)mats * M * N[i];
+    int cfg = 0, ks = 1;
+    double best = 0.0;
+    for (int c = 0; c < 3; c++) {
+        const PTile &t = kPTiles[c];
+        const int tno = t.tn / mats;
+        long long tiles = 0;
+        for (int i = 0; i < nseg; i++) tiles += (N[i] + tno - 1) / tno;
+        tiles *= (M + t.tm - 1) / t.tm;
+        for (int k = 1; k <= 16 && k <= K / 256; k *= 2) {
+            if (k > 1 && msum * k > part_floats) break;
+            static const double one[] = {1.68, 0.85, 0.6}, full[] = {2.43, 1.49, 0.8};
+            const long long wgs = tiles * k, slots = 256 * t.per_cu, rounds = (wgs + slots - 1) / slots;
+            const double stages = 8.0 * ((K / 256 + k - 1) / k);
+            const double cost = rounds * (stages * (wgs <= 256 ? one[c] : full[c]) + 6.0) +
+                                (k > 1 ? 4.0 + (double)msum * 4.0 * (2 * k + 1) / 3.0e6 : 0.0);
+            if (best == 0.0 || cost < best) best = cost, cfg = c, ks = k;
+        }
+    }
+    return {cfg, ks};
+}
+
 bool pgemm_supported(int fmt, int K, const void *w, uint64_t stride) {
     return qgemm_enabled() && qgemm_supported(fmt, K, w, nullptr, stride, 0);
 }
@@ -587,24 +614,7 @@ hipError_t launch_pgemm(int fmt, int nseg, const uint8_t *const *w, const uint8_
     p.stride = stride;
     p.x = xp.x, p.xs = xp.xs, p.xscale = xp.scale;
     p.M = M, p.K = K;
-    int cfg = 0, ks = 1;
-    double best = 0.0;
-    for (int c = 0; c < 3; c++) {
-        const PTile &t = kPTiles[c];
-        const int tno = t.tn / mats;
-        long long tiles = 0;
-        for (int i = 0; i < nseg; i++) tiles += (N[i] + tno - 1) / tno;
-        tiles *= (M + t.tm - 1) / t.tm;
-        for (int k = 1; k <= 16 && k <= K / 256; k *= 2) {
-            if (k > 1 && (!part || p.msum * k > part_floats)) break;
-            static const double one[] = {1.68, 0.85, 0.6}, full[] = {2.43, 1.49, 0.8};
-            const long long wgs = tiles * k, slots = 256 * t.per_cu, rounds = (wgs + slots - 1) / slots;
-            const double stages = 8.0 * ((K / 256 + k - 1) / k);
-            const double cost = rounds * (stages * (wgs <= 256 ? one[c] : full[c]) + 6.0) +
-                                (k > 1 ? 4.0 + (double)p.msum * 4.0 * (2 * k + 1) / 3.0e6 : 0.0);
-            if (best == 0.0 || cost < best) best = cost, cfg = c, ks = k;
-        }
-    }
+    const auto [cfg, ks] = pgemm_plan(nseg, N, M, K, mats, part ? part_floats : 0);
     const PTile &t = kPTiles[cfg];
     int nt = 0;
     for (int i = 0; i < 3; i++) {
@@ -746,3 +756,22 @@ hipError_t launch_norm_planes(const float *x, const float *w, float *out, int ro
 }
 
 }  // namespace zh
+
+extern "C" int ziggy_hip_probe_prompt_tiles(const uint32_t *rows, uint32_t count, uint32_t tokens, uint32_t cols, int pair,
+                                            size_t workspace_floats, ZiggyHipPromptTiles *out, char *err, size_t err_len) {
+    bool ok = rows && out && count >= 1 && count <= 3 && (!pair || count == 1) && tokens >= 1 && tokens <= 1u << 20 &&
+              cols >= 256 && cols % 256 == 0 && cols <= 1u << 20;
+    int n[3] = {};
+    for (uint32_t i = 0; ok && i < count; i++) {
+        ok = rows[i] >= 1 && rows[i] <= 1u << 20;
+        n[i] = (int)rows[i];
+    }
+    if (!ok) {
+        zh::set_err(err, err_len, "invalid probe_prompt_tiles arguments");
+        return ZIGGY_HIP_INVALID_ARGUMENT;
+    }
+    const zh::PgPlan plan = zh::pgemm_plan((int)count, n, (int)tokens, (int)cols, pair ? 2 : 1, workspace_floats);
+    const zh::PTile &t = zh::kPTiles[plan.cfg];
+    *out = {(uint32_t)t.tm, (uint32_t)t.tn, (uint32_t)plan.ks};
+    return ZIGGY_HIP_OK;
+}

@@ -74,6 +74,10 @@ class RowLoadProbe(ctypes.Structure):
                 ("slot_us", ctypes.c_double * 2), ("coalesced_us", ctypes.c_double * 2), ("lds_us", ctypes.c_double * 2)]
 
 
+class PromptTiles(ctypes.Structure):
+    _fields_ = [("tokens", ctypes.c_uint32), ("rows", ctypes.c_uint32), ("split", ctypes.c_uint32)]
+
+
 class GenerateStats(ctypes.Structure):
     _fields_ = [("steps", ctypes.c_uint64), ("gpu_elapsed_ns", ctypes.c_uint64), ("wall_ns", ctypes.c_uint64),
                 ("next_token", ctypes.c_uint32), ("reserved", ctypes.c_uint32), ("prompt_ns", ctypes.c_uint64)]
@@ -152,6 +156,7 @@ def lib() -> ctypes.CDLL:
         "ziggy_hip_probe_chain": [vp, vp, u32, u32, ctypes.POINTER(ChainProbe)] + E,
         "ziggy_hip_probe_sync": [vp, u32, ctypes.POINTER(SyncProbe)] + E,
         "ziggy_hip_probe_row_load": [vp, u32, ctypes.POINTER(RowLoadProbe)] + E,
+        "ziggy_hip_probe_prompt_tiles": [vp, u32, u32, u32, i, sz, ctypes.POINTER(PromptTiles)] + E,
         "ziggy_hip_indexed_matvec": [vp, u32, vp, vp, vp, u32, u32, vp, u32, u32, i] + E,
         "ziggy_hip_run_gemm": [vp, u32, vp, vp, vp, u32, u32, u32, i] + E,
         "ziggy_hip_dual_indexed_matvec": [vp, u32, vp, vp, vp, vp, vp, u32, u32, vp, u32, u32] + E,
@@ -258,6 +263,14 @@ class Buffer:
             self.free()
         except Exception:
             pass
+
+
+def prompt_tiles(rows, tokens: int, cols: int, pair: bool = False, workspace: int = 16 << 20):
+    """(tokens, rows, split) of a prompt product's tiles (ziggy_hip_probe_prompt_tiles)."""
+    r = np.ascontiguousarray(rows, np.uint32)
+    out = PromptTiles()
+    _call("ziggy_hip_probe_prompt_tiles", r.ctypes.data, r.size, tokens, cols, int(pair), workspace, ctypes.byref(out))
+    return out.tokens, out.rows, out.split
 
 
 class Context:
