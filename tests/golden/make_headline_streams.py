@@ -9,8 +9,8 @@ CPU decode path, fed token by token as runPrompt does, model/loader.zig:1016-103
   * `f32_kv`: the same prompt and 64 tokens with an f32 KV cache, the reference CPU path proper
     (model/loader.zig:950-951), and the first step where it leaves the binary16 stream (null: none);
   * `long`: a 320-token seeded prompt (binary16 KV), the logits after it (in the .npz) and the next 64
-    greedy tokens.  The HIP session runs such a prompt in batched passes of up to 256 rows, so this
-    pins its two-token-tile GEMMs over full reductions (K = 4096 and 14336 / 12288).  The entry also
+    greedy tokens.  The HIP session runs such a prompt in one batched pass, so this
+    pins its prompt products over full reductions (K = 4096 and 14336 / 12288).  The entry also
     records the oracle's own sensitivity there: the relative L2 change of its logits when one weight of
     layer 0's attention norm moves by one ulp.
 The oracle needs minutes for these on host cores, so they are computed once here and the GPU tests

@@ -12,8 +12,8 @@ semantics):
     the same argmax, logits within 1e-4 relative L2;
   * Qwen3: one batched verify pass of the pending token and 8 drafts (M = 9 GEMMs on the matrix cores)
     predicts the oracle's greedy continuation, after the prompt and over a 2048-row filled cache;
-  * a 320-token prompt, which the session runs in batched passes of up to 256 rows (the two-token-tile
-    split-input GEMMs over the full reductions, K = 4096 and 14336 / 12288): the logits after it
+  * a 320-token prompt, which the session runs in one batched pass (319 rows of the prompt products over
+    the full reductions, K = 4096 and 14336 / 12288): the logits after it
     against the oracle's (tests/golden/headline_long_logits.npz) and the next 64 greedy tokens;
   * the reference CPU path proper keeps an f32 KV cache (model/loader.zig:950-951): the HIP stream
     against the oracle's f32-KV stream, which must leave it at the step the fixture records (none

@@ -1,11 +1,12 @@
 """Batched prompt prefill on the matrix cores against the oracle's token-by-token prompt.
 
 The reference feeds a prompt one token at a time (runPrompt, model/loader.zig:1016-1036); the session
-runs every prompt token but the last in batched passes of up to 256 tokens (exact-code GEMMs, multi-query
+runs every prompt token but the last in batched passes of up to 4096 tokens (exact-code products, tiled
 causal attention over the rows the pass itself stores), then the last one through the decode step.  The
 logits after the prompt must be within 1e-4 relative L2 of the oracle's, and the next 64 greedy tokens
-equal its stream.  Prompts of 300 tokens take two passes, the last one ragged; the models cover query
-heads per kv head 1, 2 and 8, head sizes 64 and 128, per-head QK norm and Q4_K_M / Q8_0 weights.
+equal its stream.  Prompts of 300 tokens end off a tile's edge (where one pass ends and the next begins:
+test_gpu_prompt_passes.py); the models cover query heads per kv head 1, 2 and 8, head sizes 64 and 128, per-head
+QK norm and Q4_K_M / Q8_0 weights.
 """
 import sys
 
@@ -36,16 +37,15 @@ MODELS = {
                               default_type=Q8_0, attn_v_type=Q8_0, output_type=Q8_0, embd_type=Q8_0, context=512,
                               rope_theta=1000000.0),
     "llama-hd96-g4": dict(arch="llama", hidden=768, ffn=1024, n_head=8, n_kv=2, head_dim=96, context=512),
-    # Q8_0 with odd chunk counts (768 and 1280 values): the two-tile product's one-chunk stages end on a
-    # chunk whose pair partner is past the range
+    # Q8_0 with odd counts of 256 values (768 and 1280): reductions that don't split evenly
     "llama-q8-odd-chunks": dict(arch="llama", hidden=768, ffn=1280, n_head=6, n_kv=2, head_dim=128,
                                 default_type=Q8_0, attn_v_type=Q8_0, output_type=Q8_0, embd_type=Q8_0, context=512),
 }
 
 
 @pytest.mark.parametrize("name", list(MODELS))
-# 18: one pass of 17 rows (the two-token-tile products with a second tile of one row); 65 and 300: full
-# and partial tiles over one or two passes
+# 2: the products of passes of up to 16 rows; 18: 17 rows, the fewest of the prompt products; 65 and 300: a
+# full tile of 64 rows, and a partial one behind four
 @pytest.mark.parametrize("plen", [2, 18, 65, 300])
 def test_batched_prefill_matches_the_token_by_token_prompt(hip_ctx, name, plen):
     say(f"prefill {name} prompt {plen}")

@@ -33,7 +33,6 @@
 // card (its clock falls to 1.95 GHz under this load); a slab takes about 4100 cycles of which the
 // matrix cores are busy 2048.  The same wait for codes and loads together took 1300 us, without
 // the asynchronous copy 1293 us with one slab in registers.
-#include <cstdlib>
 #include <type_traits>
 
 #include "zh_internal.h"
@@ -93,8 +92,7 @@ template <> struct PFmt<Q4_K> {
         float m[8];
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            const uint32_t lo = (hd.y >> (8 * j)) & 0xFFu, mid = (hd.z >> (8 * j)) & 0xFFu, top = (hd.w >> (8 * j)) & 0xFFu;
-            (void)lo;
+            const uint32_t mid = (hd.z >> (8 * j)) & 0xFFu, top = (hd.w >> (8 * j)) & 0xFFu;
             m[j] = live ? -64.f * (float)(mid & 63) : 0.f;
             m[4 + j] = live ? -64.f * (float)((top >> 4) | ((mid >> 6) << 4)) : 0.f;
         }
@@ -538,8 +536,13 @@ typedef void (*PGemmKernel)(PGemmParams);
 // reduction is split over up to 16 workgroups (partial results added by a second launch in a
 // fixed order).  The choice is the least estimate of time: rounds of workgroups over the chip x
 // slabs x the measured time of a slab (us; alone on a CU, and with the CU shared or the whole chip
-// busy), 6 us for the launch, and the partial results' traffic.  Measured, 76 / 256 / 600 / 1200
-// rows x (4096 x 4096, Q4_K): 28.1 / 43.7 / 90 / 150 us chosen or within 8%, one tile size 211-229 us.
+// busy), 6 us for the launch, and the partial results' traffic.  The slab times are Q4_K's; a format
+// with a third product per code (Q6_K, IQ4_XS) scales them alike.  Measured against every tile and
+// split, 76 / 256 / 600 / 1200 / 4095 rows: 4096 x 4096 Q4_K 29 / 41 / 82 / 128 / 260 us, within 3% of
+// the best, Q6_K 33 / 50 / 108 / 188 / 369 and IQ4_XS 31 / 48 / 105 / 173 / 353 within 5%, Q8_0 7%, Q3_K
+// 12% (256 rows).  1024 x 4096: within 11% up to 256 rows, 7-19% at 600 and 1200; at 4095 rows 64 x 128
+// unsplit is taken where 256 x 256 in four parts would be 1.14-1.33 times as fast (the estimate
+// charges the partial results too much there).
 struct PTile {
     int tm, tn, threads, per_cu;  // tile, workgroup size, workgroups that share a CU
 };

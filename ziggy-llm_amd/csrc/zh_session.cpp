@@ -1191,11 +1191,12 @@ static hipError_t pass_enqueue(ZiggyHipSession *s, const uint32_t *tokens, int M
     const float eps = md.rms_norm_eps;
     hipError_t e = launch_embed_rows(tokens, M, s->embd.p, s->embd.stride, (int)s->embd.rows, s->embd.type, H,
                                      s->b_hidden, st);
-    // Prompt chunks are deterministic: no reduction split onto the residual,
-    // at most two onto cleared rows (0 + a + b is the same sum in either
-    // order), none for gate/up, which store their rows; their token tiles
-    // fill the chip.  Verify passes (one token
-    // tile) keep the split for speed; their sums vary in the last bits.
+    // Prompt chunks are deterministic.  The products from planes (below) add
+    // the parts of a split in a fixed order.  The others split no reduction
+    // onto the residual, at most in two onto cleared rows (0 + a + b is the
+    // same sum in either order), and none for gate/up, which store their
+    // rows.  Verify passes (one token tile) split freely, for speed; their
+    // sums vary in the last bits.
     const bool det = !output;
     // ZIGGY_HIP_VERIFY_SPLIT: the verify pass's largest reduction split (a tuning knob)
     static const int vsplit = [] {
